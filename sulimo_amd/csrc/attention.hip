@@ -799,7 +799,11 @@ int32_t launch_hd(const AttnArgs &a, hipStream_t s) {
     // kept window: the earlier positions not yet valid (and, unless the caller wrote
     // them, the ubatch's own), nothing past the last position
     const int jn0 = a.start_pos;
-    const int end = a.win_new_done ? (jn0 + kWinKeys - 1) / kWinKeys : (w.len + kWinKeys - 1) / kWinKeys;
+    // (nothing to do when every earlier position is valid and the caller wrote its own,
+    // also where the ubatch starts inside a block: 5 us per layer of a short chat turn)
+    const int end = !a.win_new_done      ? (w.len + kWinKeys - 1) / kWinKeys
+                    : a.win_valid >= jn0 ? 0
+                                         : (jn0 + kWinKeys - 1) / kWinKeys;
     if ((rc = window_blocks(std::min(a.win_valid, jn0) / kWinKeys, end))) return rc;
   } else if (a.win_new_done) {
     const int jn0 = (int)(a.start_pos - w.lo);  // window index of the first new position

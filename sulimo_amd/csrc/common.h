@@ -259,6 +259,14 @@ int32_t launch_gemm_q4_0(const GemmArgs &a, hipStream_t s, bool *norm_done = nul
 // Partial-sum workspace launch_gemm_q4_0 would use for this GEMM given unlimited room.
 size_t gemm_q4_0_workspace_bytes(const GemmArgs &a);
 
+// The GEMM for a handful of tokens (gemm_skinny.hip), chosen inside launch_gemm_q4_0:
+// whether it takes the call, the K splits it would use (1: the epilogue runs in the
+// kernel), and the launch itself, with EPI_PART and a.splits for the f32 partials of a split.
+constexpr int kSkinnyMaxTokens = 64, kSkinnyMaxRopeTokens = 48;
+bool skinny_fits(const GemmArgs &a);
+int skinny_splits(const GemmArgs &a, bool unbounded);
+int32_t launch_skinny(const GemmArgs &a, hipStream_t s, LaunchStamp st);
+
 // Size of the static device scratch array of the no-alloc GEMM entry point (one per
 // device, held until the process ends).
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;

@@ -37,138 +37,10 @@
 #include <utility>
 
 #include "common.h"
+#include "q4_mfma.h"
 
 namespace sulimo {
 namespace {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-
-constexpr int kBK = 64;                   // k per stage
-constexpr uint32_t kOob = 0x80000000u;    // buffer offset past every buffer: reads as zero
-constexpr uint32_t kRsrcWord3 = 0x00020000u;  // raw buffer, 32-bit data format (gfx9)
-constexpr int kXcds = 8;                      // XCDs of an MI355X
-
-template <int J>
-using ic = std::integral_constant<int, J>;
-
-template <typename F, int... J>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, J...>) {
-  (f(ic<J>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-
-__device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, (int)kRsrcWord3);
-}
-
-// One buffer -> LDS DMA: active lane i writes 16 bytes at dst + 16*i.
-__device__ __forceinline__ void dma16(rsrc_t r, void *dst, uint32_t voff, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)dst, 16, (int)voff, soff, 0, 0);
-}
-
-// Four nibbles, one per byte in bits [3:0] (HI = false) or [7:4] (HI = true) with the
-// other bits clear -> two half2 of (q-8)*d.
-template <bool HI>
-__device__ __forceinline__ void dq4(uint32_t nib, half2v d2, half2v &a, half2v &b) {
-  // bytes [n0, 0x64, n1, 0x64] -> half2(1024 + n0, 1024 + n1), exact
-  const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u);
-  const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u);
-  if constexpr (HI) {  // 1024 + 16q: /16 - 72 = q - 8, one exact fma
-    const half2v s = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const half2v o = {(_Float16)-72.0f, (_Float16)-72.0f};
-    a = __builtin_elementwise_fma(as_h2(p0), s, o) * d2;
-    b = __builtin_elementwise_fma(as_h2(p1), s, o) * d2;
-  } else {
-    const half2v o = {(_Float16)1032.0f, (_Float16)1032.0f};
-    a = (as_h2(p0) - o) * d2;
-    b = (as_h2(p1) - o) * d2;
-  }
-}
-
-// The same four nibbles -> two half2 of q-8 (exact, unscaled).
-template <bool HI>
-__device__ __forceinline__ void dq4_raw(uint32_t nib, half2v &a, half2v &b) {
-  const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u);
-  const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u);
-  if constexpr (HI) {
-    const half2v s = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const half2v o = {(_Float16)-72.0f, (_Float16)-72.0f};
-    a = __builtin_elementwise_fma(as_h2(p0), s, o);
-    b = __builtin_elementwise_fma(as_h2(p1), s, o);
-  } else {
-    const half2v o = {(_Float16)1032.0f, (_Float16)1032.0f};
-    a = as_h2(p0) - o;
-    b = as_h2(p1) - o;
-  }
-}
-
-// s_waitcnt vmcnt(n) with expcnt and lgkmcnt left unconstrained (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-// Workgroup barrier that orders LDS accesses only: global loads and stores in flight
-// stay in flight (__syncthreads also waits for those).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Lane exchanges within a quad of lanes (DPP quad_perm): partner lane j^1, j^2.
-__device__ __forceinline__ uint32_t dpp_xor1(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);
-}
-__device__ __forceinline__ uint32_t dpp_xor2(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);
-}
-__device__ __forceinline__ uint32_t fu(float v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ __forceinline__ float uf(uint32_t v) { return __builtin_bit_cast(float, v); }
-
-// 4 x 4 transposes across a lane quad. Lane j of the quad holds rows 0..3 of column j;
-// afterwards it holds row j, columns 0..3. Every lane of the quad must be active.
-// f16: p = rows 0,1 and q = rows 2,3 (packed); returns columns 0,1 and 2,3 (packed).
-__device__ __forceinline__ uint2 quad_t16(uint32_t p, uint32_t q, int j) {
-  const uint32_t sel = (j & 1) ? 0x03020706u : 0x05040100u;
-  const uint32_t x = __builtin_amdgcn_perm(dpp_xor1(p), p, sel);  // row j&1 (odd) or 0, columns pair of j
-  const uint32_t y = __builtin_amdgcn_perm(dpp_xor1(q), q, sel);  // row 2 + (j&1)
-  const uint32_t r = dpp_xor2((j & 2) ? x : y);
-  return (j & 2) ? uint2{r, y} : uint2{x, r};
-}
-__device__ __forceinline__ float4 quad_t32(float a0, float a1, float a2, float a3, int j) {
-  const bool odd = j & 1, h = j & 2;
-  const float r1 = uf(dpp_xor1(fu(odd ? a0 : a1)));
-  const float r2 = uf(dpp_xor1(fu(odd ? a2 : a3)));
-  const float x0 = odd ? r1 : a0, x1 = odd ? a1 : r1;  // row j&1, the pair of columns holding j
-  const float y0 = odd ? r2 : a2, y1 = odd ? a3 : r2;  // row 2 + (j&1)
-  const float t0 = uf(dpp_xor2(fu(h ? x0 : y0))), t1 = uf(dpp_xor2(fu(h ? x1 : y1)));
-  return h ? float4{t0, t1, y0, y1} : float4{x0, x1, t0, t1};
-}
-// Four consecutive K-split partials as f32, stored as f16 or f32.
-template <bool F16>
-__device__ __forceinline__ float4 load_part4(const float *part, size_t idx) {
-  if constexpr (F16) {
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    const h4 v = *reinterpret_cast<const h4 *>(reinterpret_cast<const _Float16 *>(part) + idx);
-    return float4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-  } else {
-    return *reinterpret_cast<const float4 *>(part + idx);
-  }
-}
-__device__ __forceinline__ uint32_t pack_h2(float lo, float hi) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
-}
 
 template <int FM, int FN, int kNS, int EPI, int KSPLIT, int WM>
 __global__ __launch_bounds__(256 * KSPLIT, (WM == 2 || KSPLIT > 1) ? 1 : 2) void gemm_q4_kernel(GemmArgs a) {
@@ -986,9 +858,9 @@ __global__ __launch_bounds__(256 * KSPLIT, (WM == 2 || KSPLIT > 1) ? 1 : 2) void
 
 // Sum of the K splits' partials in split order (deterministic), then the real epilogue:
 // one thread per 4 consecutive columns of the concatenated segment columns of a row.
-template <int EPI>
+// F16: f16 partials.
+template <int EPI, bool F16>
 __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs a) {
-  constexpr bool kF16 = EPI != EPI_F32;  // partials at the output's precision
   const int c4 = a.ldp / 4;
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= (long)a.m * c4) return;
@@ -996,9 +868,9 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs a) {
   int col = (int)(gid - (long)row * c4) * 4;
   const size_t plane = (size_t)a.m * a.ldp;
   const size_t p = (size_t)row * a.ldp + col;
-  float4 v = load_part4<kF16>(a.part, p);
+  float4 v = load_part4<F16>(a.part, p);
   for (int s = 1; s < a.splits; s++) {
-    const float4 w = load_part4<kF16>(a.part, p + s * plane);
+    const float4 w = load_part4<F16>(a.part, p + s * plane);
     v.x += w.x;
     v.y += w.y;
     v.z += w.z;
@@ -1096,18 +968,59 @@ __global__ __launch_bounds__(256) void split_reduce_norm_vec_kernel(GemmArgs a) 
   }
 }
 
+// The same for the few rows of a skinny GEMM (f32 partials, at most 8 splits): one
+// workgroup per row, one wave per 256 columns with every load of the row in flight at
+// once. The row meets in LDS, where each wave sums its squares in the one-wave order, so
+// residual and normed bytes equal those of the separate kernels here too.
+template <int V>
+__global__ __launch_bounds__(64 * V) void split_reduce_norm_rows_kernel(GemmArgs a) {
+  constexpr int D = 256 * V, kSplits = 8;
+  __shared__ float4 xs[64 * V];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, c = 4 * threadIdx.x;
+  const GemmSegment seg = a.seg[0];
+  const size_t plane = (size_t)a.m * a.ldp;
+  const size_t p = (size_t)row * a.ldp + c;
+  float *x = reinterpret_cast<float *>(seg.out) + (size_t)row * seg.ldo + c;
+  const float4 nw = *reinterpret_cast<const float4 *>(a.norm_w + c);
+  const float4 old = *reinterpret_cast<const float4 *>(x);
+  const float4 b = seg.bias ? *reinterpret_cast<const float4 *>(seg.bias + c) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 w[kSplits];  // splits past the last repeat it, not added below
+#pragma unroll
+  for (int sp = 0; sp < kSplits; sp++) w[sp] = load_part4<false>(a.part, p + min(sp, a.splits - 1) * plane);
+  float4 v = w[0];
+#pragma unroll
+  for (int sp = 1; sp < kSplits; sp++) {
+    if (sp < a.splits) v = float4{v.x + w[sp].x, v.y + w[sp].y, v.z + w[sp].z, v.w + w[sp].w};
+  }
+  if (seg.bias) v = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
+  const float4 nx = float4{old.x + (float)(_Float16)v.x, old.y + (float)(_Float16)v.y, old.z + (float)(_Float16)v.z,
+                           old.w + (float)(_Float16)v.w};
+  *reinterpret_cast<float4 *>(x) = nx;
+  xs[threadIdx.x] = nx;
+  lds_barrier();
+  float ss = 0.0f;
+#pragma unroll
+  for (int j = 0; j < V; j++) ss = rms_sumsq4(xs[64 * j + lane], ss);
+  const float scale = rms_scale(rms_wave_sum(ss), D, a.norm_eps);
+  const size_t o = (size_t)row * D + c;
+  *reinterpret_cast<rms_half4 *>(reinterpret_cast<_Float16 *>(a.norm_out) + o) = rms_out4(nx, scale, nw);
+  if (a.norm_x16)
+    *reinterpret_cast<rms_half4 *>(reinterpret_cast<_Float16 *>(a.norm_x16) + o) =
+        rms_half4{(_Float16)nx.x, (_Float16)nx.y, (_Float16)nx.z, (_Float16)nx.w};
+}
+
 // K-split reduction of an EPI_RESID GEMM fused with the RMSNorm of the rows it updates:
 // one workgroup per row holding its V*1024 columns in registers. x += f16(partials summed
 // in split order (+ bias)), as split_reduce_kernel does, then norm_out = f16(x * scale *
 // norm_w) with scale = 1 / sqrt(mean(x^2) + eps), and norm_x16 = f16(x) when set.
-template <int V>
+template <int V, bool F16>
 __global__ __launch_bounds__(256) void split_reduce_norm_kernel(GemmArgs a) {
   typedef _Float16 half4v __attribute__((ext_vector_type(4)));
   const int row = blockIdx.x, tid = threadIdx.x;
   const GemmSegment seg = a.seg[0];
   const int n4 = seg.n / 4;
   const size_t plane = (size_t)a.m * a.ldp;
-  const size_t p = (size_t)row * a.ldp;  // f16 partials (a residual GEMM's output is f16)
+  const size_t p = (size_t)row * a.ldp;
   float *x = reinterpret_cast<float *>(seg.out) + (size_t)row * seg.ldo;
   // the norm weights are loaded first: loaded between the stores at the end, each load
   // would wait for the stores before it (loads and stores retire in issue order)
@@ -1120,9 +1033,9 @@ __global__ __launch_bounds__(256) void split_reduce_norm_kernel(GemmArgs a) {
     const int c4 = tid + 256 * j;
     xv[j] = float4{0.0f, 0.0f, 0.0f, 0.0f};
     if (c4 >= n4) continue;
-    float4 v = load_part4<true>(a.part, p + 4 * c4);
+    float4 v = load_part4<F16>(a.part, p + 4 * c4);
     for (int sp = 1; sp < a.splits; sp++) {
-      const float4 w = load_part4<true>(a.part, p + sp * plane + 4 * c4);
+      const float4 w = load_part4<F16>(a.part, p + sp * plane + 4 * c4);
       v.x += w.x;
       v.y += w.y;
       v.z += w.z;
@@ -1537,6 +1450,10 @@ int32_t launch_plan(const GemmArgs &a, int cfg, hipStream_t s, LaunchStamp st) {
 size_t gemm_q4_0_workspace_bytes(const GemmArgs &a) {
   if (a.m <= 0 || a.k <= 0 || a.k % 32 != 0 || a.nseg < 1 || a.nseg > 3) return 0;
   if (gemv_fits(a)) return 0;
+  if (skinny_fits(a)) {
+    const int splits = skinny_splits(a, true);
+    return splits > 1 ? (size_t)splits * a.m * seg_cols(a) * 4 : 0;
+  }
   const GemmPlan p = plan_gemm(a, true);
   return p.splits > 1 ? (size_t)p.splits * a.m * seg_cols(a) * part_elem_bytes(a) : 0;
 }
@@ -1578,28 +1495,34 @@ int32_t launch_gemm_q4_0(const GemmArgs &a, hipStream_t s, bool *norm_done, cons
   }
   const LaunchStamp st = stamp ? *stamp : LaunchStamp{};
   if (gemv_fits(a)) return launch_gemv(a, s, st);
-  const GemmPlan p = plan_gemm(a, false);
-  if (p.splits == 1) return launch_plan(a, p.cfg, s, st);
+  const bool skinny = skinny_fits(a);
+  const GemmPlan p = skinny ? GemmPlan{kNumCfg, skinny_splits(a, false)} : plan_gemm(a, false);
+  if (p.splits == 1) return skinny ? launch_skinny(a, s, st) : launch_plan(a, p.cfg, s, st);
   // K split: partials per split, then their sum in split order with the epilogue
   GemmArgs g = a;
   g.epi = EPI_PART;
   g.splits = p.splits;
   g.ldp = seg_cols(a);
-  g.part_f16 = part_elem_bytes(a) == 2;
-  int32_t rc = launch_plan(g, p.cfg, s, LaunchStamp{st.start, nullptr});
+  g.part_f16 = !skinny && part_elem_bytes(a) == 2;
+  const LaunchStamp st0{st.start, nullptr};
+  int32_t rc = skinny ? launch_skinny(g, s, st0) : launch_plan(g, p.cfg, s, st0);
   if (rc) return rc;
   GemmArgs r = g;
   r.epi = a.epi;
-  r.splits = normalize_splits(a.k, p.splits, &r.split_stages);
+  if (!skinny) r.splits = normalize_splits(a.k, p.splits, &r.split_stages);
   // the residual update and the RMSNorm of its rows in one pass, rows up to 8192 wide
   const int v4 = (a.seg[0].n / 4 + 255) / 256;
   if (norm_done && a.epi == EPI_RESID && a.norm_w && a.norm_out && a.nseg == 1 && a.seg[0].col0 == 0 && v4 <= 8) {
     const int n = a.seg[0].n;
-    if (n % 256 == 0 && n <= 256 * 16) {  // one wave per row
-      const dim3 grid((unsigned)((a.m + 3) / 4)), block(256);
+    if (n % 256 == 0 && n <= 256 * 16) {
+      const dim3 grid((unsigned)((a.m + 3) / 4)), block(256);  // one wave per row
       switch (n / 256) {
-#define SULIMO_SRN_CASE(V) \
-  case V: launch_stamped(split_reduce_norm_vec_kernel<V>, grid, block, 0, s, nullptr, st.stop, r); break;
+#define SULIMO_SRN_CASE(V)                                                                                   \
+  case V:                                                                                                    \
+    if (skinny)                                                                                              \
+      launch_stamped(split_reduce_norm_rows_kernel<V>, dim3((unsigned)a.m), dim3(64 * V), 0, s, nullptr, st.stop, r); \
+    else launch_stamped(split_reduce_norm_vec_kernel<V>, grid, block, 0, s, nullptr, st.stop, r);            \
+    break;
         SULIMO_SRN_CASE(1) SULIMO_SRN_CASE(2) SULIMO_SRN_CASE(3) SULIMO_SRN_CASE(4) SULIMO_SRN_CASE(5)
         SULIMO_SRN_CASE(6) SULIMO_SRN_CASE(7) SULIMO_SRN_CASE(8) SULIMO_SRN_CASE(9) SULIMO_SRN_CASE(10)
         SULIMO_SRN_CASE(11) SULIMO_SRN_CASE(12) SULIMO_SRN_CASE(13) SULIMO_SRN_CASE(14) SULIMO_SRN_CASE(15)
@@ -1607,17 +1530,21 @@ int32_t launch_gemm_q4_0(const GemmArgs &a, hipStream_t s, bool *norm_done, cons
 #undef SULIMO_SRN_CASE
       }
       const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return hip_fail(e, "split_reduce_norm_vec_kernel launch");
+      if (e != hipSuccess) return hip_fail(e, "K-split reduction with RMSNorm launch");
       *norm_done = true;
       return SULIMO_HIP_OK;
     }
     const dim3 grid((unsigned)a.m), block(256);
+    auto norm = [&](auto k32, auto k16) {
+      if (skinny) launch_stamped(k32, grid, block, 0, s, nullptr, st.stop, r);
+      else launch_stamped(k16, grid, block, 0, s, nullptr, st.stop, r);
+    };
     switch (v4) {
-      case 1: launch_stamped(split_reduce_norm_kernel<1>, grid, block, 0, s, nullptr, st.stop, r); break;
-      case 2: launch_stamped(split_reduce_norm_kernel<2>, grid, block, 0, s, nullptr, st.stop, r); break;
-      case 3: launch_stamped(split_reduce_norm_kernel<3>, grid, block, 0, s, nullptr, st.stop, r); break;
-      case 4: launch_stamped(split_reduce_norm_kernel<4>, grid, block, 0, s, nullptr, st.stop, r); break;
-      default: launch_stamped(split_reduce_norm_kernel<8>, grid, block, 0, s, nullptr, st.stop, r); break;
+      case 1: norm(split_reduce_norm_kernel<1, false>, split_reduce_norm_kernel<1, true>); break;
+      case 2: norm(split_reduce_norm_kernel<2, false>, split_reduce_norm_kernel<2, true>); break;
+      case 3: norm(split_reduce_norm_kernel<3, false>, split_reduce_norm_kernel<3, true>); break;
+      case 4: norm(split_reduce_norm_kernel<4, false>, split_reduce_norm_kernel<4, true>); break;
+      default: norm(split_reduce_norm_kernel<8, false>, split_reduce_norm_kernel<8, true>); break;
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "split_reduce_norm_kernel launch");
@@ -1627,9 +1554,15 @@ int32_t launch_gemm_q4_0(const GemmArgs &a, hipStream_t s, bool *norm_done, cons
   const long threads = (long)a.m * (r.ldp / 4);
   const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
   switch (a.epi) {
-    case EPI_F16: launch_stamped(split_reduce_kernel<EPI_F16>, grid, block, 0, s, nullptr, st.stop, r); break;
-    case EPI_F32: launch_stamped(split_reduce_kernel<EPI_F32>, grid, block, 0, s, nullptr, st.stop, r); break;
-    default: launch_stamped(split_reduce_kernel<EPI_RESID>, grid, block, 0, s, nullptr, st.stop, r); break;
+    case EPI_F16:
+      if (skinny) launch_stamped(split_reduce_kernel<EPI_F16, false>, grid, block, 0, s, nullptr, st.stop, r);
+      else launch_stamped(split_reduce_kernel<EPI_F16, true>, grid, block, 0, s, nullptr, st.stop, r);
+      break;
+    case EPI_F32: launch_stamped(split_reduce_kernel<EPI_F32, false>, grid, block, 0, s, nullptr, st.stop, r); break;
+    default:
+      if (skinny) launch_stamped(split_reduce_kernel<EPI_RESID, false>, grid, block, 0, s, nullptr, st.stop, r);
+      else launch_stamped(split_reduce_kernel<EPI_RESID, true>, grid, block, 0, s, nullptr, st.stop, r);
+      break;
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SULIMO_HIP_OK : hip_fail(e, "split_reduce_kernel launch");
