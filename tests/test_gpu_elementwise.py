@@ -1,0 +1,51 @@
+"""GPU: the bandwidth operations' vector forms at their edges: totals around a thread's 8
+elements, head counts that do not fill a RoPE thread's group of 4, partial rotation, and
+rotation widths that take the element-wise kernel."""
+import numpy as np
+import pytest
+
+import oracle
+from sulimo_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+
+def up(ctx, a):
+    return hip.HipBuffer.from_host(ctx, np.ascontiguousarray(a))
+
+
+@pytest.mark.parametrize("total", [1, 7, 8, 9, 2047, 2048, 2049])
+def test_silu_and_add_edges(ctx, total):
+    rng = np.random.default_rng(total)
+    g, u = ((rng.standard_normal(total + 8) * s).astype(np.float16) for s in (3, 1))
+    ob = up(ctx, g)
+    hip.enqueue_silu_mul(ctx, up(ctx, g), up(ctx, u), ob, total)
+    got = ob.download(np.float16, g.shape)
+    want = oracle.cl_silu_mul_f16(g[:total], u[:total]).astype(np.float64)
+    # hardware exp2 and reciprocal (a few f32 ulps), then one f16 rounding
+    assert np.all(np.abs(got[:total] - want) <= 1.01 * np.spacing(np.abs(want).astype(np.float16)).astype(np.float64))
+    assert np.array_equal(got[total:], g[total:])  # nothing past the end is written
+    ab = up(ctx, g)
+    hip.enqueue_add(ctx, ab, up(ctx, u), total)
+    got = ab.download(np.float16, g.shape)
+    assert np.array_equal(got[:total], oracle.cl_add_f16(g[:total], u[:total]))
+    assert np.array_equal(got[total:], g[total:])
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("heads,hd,rd,n", [(5, 64, 40, 3), (1, 128, 128, 1), (7, 64, 12, 5), (9, 32, 32, 70)])
+def test_rope_partial_heads_and_widths(ctx, mode, heads, hd, rd, n):
+    """Bit for bit given the device's cos/sin table (products rounded before the add)."""
+    rng = np.random.default_rng(heads + rd + n)
+    v = rng.standard_normal((n, heads, hd)).astype(np.float16)
+    vb, tb = up(ctx, v), hip.HipBuffer.device_only(ctx, n * rd // 2 * 8)
+    hip.enqueue_rope(ctx, vb, heads, hd, rd, 1e4, mode, 11, n)
+    hip.rope_table(ctx, rd, 1e4, 11, n, tb)
+    tab = tb.download(np.float32, (n, 1, rd // 2, 2))
+    i = np.arange(rd // 2)
+    i0, i1 = (2 * i, 2 * i + 1) if mode == 0 else (i, i + rd // 2)
+    x = v.astype(np.float32)
+    want = x.copy()
+    want[:, :, i0] = x[:, :, i0] * tab[..., 0] - x[:, :, i1] * tab[..., 1]
+    want[:, :, i1] = x[:, :, i0] * tab[..., 1] + x[:, :, i1] * tab[..., 0]
+    assert np.array_equal(vb.download(np.float16, v.shape).view(np.uint16), want.astype(np.float16).view(np.uint16))
