@@ -266,6 +266,9 @@ constexpr int kSkinnyMaxTokens = 64, kSkinnyMaxRopeTokens = 48;
 bool skinny_fits(const GemmArgs &a);
 int skinny_splits(const GemmArgs &a, bool unbounded);
 int32_t launch_skinny(const GemmArgs &a, hipStream_t s, LaunchStamp st);
+// The same reading the weights from the source arrays (scales [n][k/32], quants
+// [n][k/32][16]): one f16 segment that skinny_fits, no panels and no workspace.
+int32_t launch_skinny_soa(const GemmArgs &a, const uint16_t *scales, const uint8_t *quants, hipStream_t s);
 
 // Size of the static device scratch array of the no-alloc GEMM entry point (one per
 // device, held until the process ends).

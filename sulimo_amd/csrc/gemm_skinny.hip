@@ -32,8 +32,8 @@
 // dequantization (60 VALU per fragment and step), and the sum over the waves.
 //
 // With SOA the weights are read from the caller's own arrays (scales [n][k/32], quants
-// [n][k/32][16]) instead of a panel copy: lane 16 g + r then holds block g of the pair's
-// four, and MFMA i takes k 32 g + 16 (i%2) + 8 (i/2) .. +7.
+// [n][k/32][16]) instead of a panel copy, the same bytes to the same lanes (two 8-byte
+// loads and two scales each), so the sums are the same bits.
 #include <algorithm>
 
 #include "common.h"
@@ -43,6 +43,7 @@ namespace sulimo {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kPairK = 128;      // k per wave step (two panel stages)
@@ -112,8 +113,9 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
 #pragma unroll
     for (int f = 0; f < NF; f++) {
       const int row = 32 * panel_of(f >> 1) + r1 + 16 * (f & 1);
-      qoff[f] = row < seg.n ? ((uint32_t)row * nb + g) * 16u : kOob;
-      soff[f] = row < seg.n ? ((uint32_t)row * nb + g) * 2u : kOob;
+      const uint32_t blk = (uint32_t)row * nb + 2u * (g >> 1);  // first block of the lane's stage
+      qoff[f] = row < seg.n ? blk * 16u + 8u * (g & 1) : kOob;
+      soff[f] = row < seg.n ? blk * 2u : kOob;
     }
   } else {
     rq = rs = make_rsrc(seg.panels, (uint32_t)npanels * (uint32_t)nst * (uint32_t)kQ4PanelRecord);
@@ -130,12 +132,17 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
   u32x4 q[NF];
   uint32_t sc[NF];
   auto load_w = [&](int pr) __attribute__((always_inline)) {
-    const bool in = SOA ? 4 * pr + g < nb : 2 * pr + (g >> 1) < nst;
+    const bool in = 2 * pr + (g >> 1) < nst;
 #pragma unroll
     for (int f = 0; f < NF; f++) {
       if constexpr (SOA) {
-        q[f] = __builtin_amdgcn_raw_buffer_load_b128(rq, in ? qoff[f] : kOob, pr * 64, 0);
-        sc[f] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, in ? soff[f] : kOob, pr * 8, 0);
+        const bool in1 = 4 * pr + 2 * (g >> 1) + 1 < nb;  // an odd block count ends in half a stage
+        const u32x2 b0 = __builtin_amdgcn_raw_buffer_load_b64(rq, in ? qoff[f] : kOob, pr * 64, 0);
+        const u32x2 b1 = __builtin_amdgcn_raw_buffer_load_b64(rq, in1 ? qoff[f] + 16u : kOob, pr * 64, 0);
+        const uint32_t s0 = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, in ? soff[f] : kOob, pr * 8, 0);
+        const uint32_t s1 = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, in1 ? soff[f] + 2u : kOob, pr * 8, 0);
+        q[f] = u32x4{b0[0], b0[1], b1[0], b1[1]};
+        sc[f] = s0 | s1 << 16;
       } else {
         q[f] = __builtin_amdgcn_raw_buffer_load_b128(rq, (in ? qoff[f >> 1] : kOob) + 256u * (f & 1),
                                                      pr * 2 * kQ4PanelRecord, 0);
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
     xrow[i] = row * (kPairK * 2);
     xsw[i] = 16 * (row & 15);
   }
-  const int c0 = 16 * (SOA ? 4 * g : 8 * (g >> 1) + (g & 1));  // MFMA 0's chunk, in bytes
+  const int c0 = 16 * (8 * (g >> 1) + (g & 1));  // MFMA 0's chunk, in bytes
   const int p0 = ks * sa.split_pairs, p1 = min(sa.npairs, p0 + sa.split_pairs);
   // X first: the wait for it leaves the weights in flight, and each fragment is multiplied
   // as its weights land.
@@ -214,13 +221,13 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
     for (int i = 0; i < MT; i++)
 #pragma unroll
       for (int s = 0; s < 4; s++) {
-        const int dc = 16 * (SOA ? 2 * (s & 1) + (s >> 1) : 4 * (s >> 1) + 2 * (s & 1));
+        const int dc = 16 * (4 * (s >> 1) + 2 * (s & 1));
         av[i][s] = *reinterpret_cast<const half8 *>(slot + xrow[i] + ((c0 + dc) ^ xsw[i]));
       }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
       const half2v dlo = as_h2(__builtin_amdgcn_perm(sc[f], sc[f], 0x01000100u));
-      const half2v dhi = SOA ? dlo : as_h2(__builtin_amdgcn_perm(sc[f], sc[f], 0x03020302u));
+      const half2v dhi = as_h2(__builtin_amdgcn_perm(sc[f], sc[f], 0x03020302u));
 #pragma unroll
       for (int s = 0; s < 4; s++) {
         const half2v d2 = s < 2 ? dlo : dhi;
@@ -528,6 +535,27 @@ int skinny_splits(const GemmArgs &a, bool unbounded) {
   return splits;
 }
 
+namespace {
+// 16 columns per workgroup while that leaves no CU a second one, else 32, else 64.
+int fragments_of(const GemmArgs &a) {
+  const int cus = device_cu_count();
+  return units_of(a, 1) <= cus ? 1 : units_of(a, 2) <= 2 * cus ? 2 : 4;
+}
+}  // namespace
+
+int32_t launch_skinny_soa(const GemmArgs &a, const uint16_t *scales, const uint8_t *quants, hipStream_t s) {
+  if (a.epi != EPI_F16 || a.nseg != 1 || !skinny_fits(a))
+    return fail(SULIMO_HIP_ERR_INVALID_ARGUMENT, "not a GEMM the skinny kernel reads from the source arrays");
+  const int nf = fragments_of(a);
+  int one = 1;
+  SkinnyArgs sa = skinny_args(a, nf, &one);
+  sa.scales = scales;
+  sa.quants = quants;
+  return nf == 1   ? launch_skinny_mt<1, EPI_F16, true>(sa, 1, s, LaunchStamp{})
+         : nf == 2 ? launch_skinny_mt<2, EPI_F16, true>(sa, 1, s, LaunchStamp{})
+                   : launch_skinny_mt<4, EPI_F16, true>(sa, 1, s, LaunchStamp{});
+}
+
 int32_t launch_skinny(const GemmArgs &a, hipStream_t s, LaunchStamp st) {
   int one = 1;
   if (a.epi == EPI_PART) {
@@ -537,9 +565,7 @@ int32_t launch_skinny(const GemmArgs &a, hipStream_t s, LaunchStamp st) {
   }
   if (a.epi == EPI_SWIGLU) return launch_skinny_mt<4, EPI_SWIGLU>(skinny_args(a, 4, &one), 1, s, st);
   if (a.epi == EPI_ROPE) return launch_skinny_mt<4, EPI_ROPE>(skinny_args(a, 4, &one), 1, s, st);
-  // 16 columns per workgroup while that leaves no CU a second one, else 32, else 64
-  const int cus = device_cu_count();
-  const int nf = units_of(a, 1) <= cus ? 1 : units_of(a, 2) <= 2 * cus ? 2 : 4;
+  const int nf = fragments_of(a);
   const SkinnyArgs sa = skinny_args(a, nf, &one);
 #define SULIMO_SKINNY(EPI)                                   \
   return nf == 1   ? launch_skinny_mt<1, EPI>(sa, 1, s, st)  \

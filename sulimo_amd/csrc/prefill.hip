@@ -169,6 +169,21 @@ int32_t sulimo_hip_enqueue_gemm_q4_0_f16_noalloc(sulimo_hip_ctx *ctx, const suli
     return fail(kInval, "the no-alloc GEMM holds at most " + std::to_string(kNoAllocScratchBytes) +
                             " bytes of weights in its GEMM layout; this matrix needs " + std::to_string(pan));
   if (n == 0) return SULIMO_HIP_OK;
+  GemmArgs a{};
+  a.x = dp<const uint16_t>(x);
+  a.m = (int)n;
+  a.k = (int)k;
+  a.ldx = (int)k;
+  a.epi = EPI_F16;
+  a.seg[0] = GemmSegment{nullptr, out->dev, (int)m, (int)m, 0};
+  a.nseg = 1;
+  // A handful of tokens (more than the GEMV's 4): the skinny kernel reads the weights where
+  // they are, in one launch, and leaves the scratch array alone (1536 x 1536 at 16 tokens:
+  // 15.5 us with the pack, the event and the tiled kernel, 4.6 so).
+  if (n > 4 && skinny_fits(a)) {
+    wrote(out);
+    return launch_skinny_soa(a, dp<const uint16_t>(scales), dp<const uint8_t>(quants), ctx->stream);
+  }
   NoAllocOrder *order = noalloc_order(ctx->device);
   if (!order) return fail(SULIMO_HIP_ERR_DRIVER, "the no-alloc ordering event was not created");
   // After the previous no-alloc call on this device, from whatever stream it came.
@@ -179,14 +194,7 @@ int32_t sulimo_hip_enqueue_gemm_q4_0_f16_noalloc(sulimo_hip_ctx *ctx, const suli
   if ((rc = launch_pack_q4_panels(dp<const uint16_t>(scales), dp<const uint8_t>(quants), nullptr, nullptr, (int)m,
                                   (int)k, scr, ctx->stream)))
     return rc;
-  GemmArgs a{};
-  a.x = dp<const uint16_t>(x);
-  a.m = (int)n;
-  a.k = (int)k;
-  a.ldx = (int)k;
-  a.epi = EPI_F16;
-  a.seg[0] = GemmSegment{scr, out->dev, (int)m, (int)m, 0};
-  a.nseg = 1;
+  a.seg[0].panels = scr;
   a.part = reinterpret_cast<float *>(scr + pan_al);
   a.part_bytes = kNoAllocScratchBytes - pan_al;
   if ((rc = launch_gemm_q4_0(a, ctx->stream))) return rc;

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
+from sulimo_amd import hip
 from sulimo_amd import synthetic as S
 from tests.helpers import max_rel_err
 from tests.test_gpu_fused import NORM_HD64, QWEN_LAYER, exact_model, run_mode
@@ -71,3 +72,20 @@ def test_epilogues_bit_exact_vs_separate_kernels(ctx, cfg, chunks, cap):
         assert np.array_equal(f["q"], p["q"])
         assert np.array_equal(f["swiglu"], p["swiglu"])
         assert np.max(np.abs(f["logits"] - p["logits"])) <= 1e-3 * np.abs(p["logits"]).max()
+
+
+@pytest.mark.parametrize("M,k,m_out", [(5, 32, 8), (16, 1536, 1536), (24, 96, 40), (33, 2080, 264), (64, 416, 9000),
+                                       (8, 4128, 72)])
+def test_no_alloc_reads_the_source_arrays(ctx, M, k, m_out):
+    """The no-alloc entry point reads the weights where they are: odd block counts, ragged
+    rows and each fragment count give the panel path's bits (where it does not split k)."""
+    rng = np.random.default_rng(M + k + m_out)
+    w = S.random_q4(rng, m_out, k)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    sb, qb, xb = (hip.HipBuffer.from_host(ctx, np.ascontiguousarray(a), True) for a in (w.scales, w.quants, x))
+    ob = hip.HipBuffer.device_only(ctx, M * m_out * 2)
+    print(f"skinny no-alloc GEMM m={M} k={k} n={m_out}", flush=True)
+    hip.enqueue_gemm_q4_0_f16_noalloc(ctx, sb, qb, xb, ob, m_out, k, M)
+    ctx.wait()
+    y = ob.download(np.uint16, (M, m_out))
+    assert np.array_equal(y, run_gemm(ctx, w.scales, w.quants, x, m_out, k, M).view(np.uint16))
