@@ -14,9 +14,9 @@
 //     [kv head][position][head_dim], V transposed [kv head][head_dim][position] with
 //     the positions of each 16-key group stored in the order the P V^T MFMA reads
 //     them (kperm). Values are f16(code * d), as the ring holds them.
-//  2. flash_attn_kernel: one workgroup = 8 wave64s. Four of them cover HG query
-//     heads of one KV head x PB blocks of 32 positions over the first half of the
-//     visible key tiles, the other four the same queries over the second half (two
+//  2. flash_attn_kernel: one workgroup = 4 or 8 wave64s. Four of them cover HG query
+//     heads of one KV head x PB blocks of 32 positions over the visible key tiles, or
+//     over the first half of them while the other four run the second half (two
 //     waves per SIMD, half the serial chain); the halves merge (m, l, O) through LDS
 //     at the end. K and V^T tiles of 64 keys stream into each half's two LDS slots by
 //     buffer DMA and are shared by its four waves. Per wave:
@@ -27,6 +27,14 @@
 //       O^T += V^T P^T  V^T (LDS) as A, P^T straight from the S^T registers as B.
 //     The running max m only moves when a tile's max exceeds it by more than 2^8, so
 //     the accumulator is rescaled on few tiles (P <= 256, exact to f16 precision).
+//     Per 32-key half tile h, the S MFMAs of h+1 and the PV MFMAs of h-1 run under the
+//     softmax of h, across tiles too (K runs one tile ahead of V); with the S MFMAs of a
+//     tile's first half and the PV MFMAs of its second left uncovered, the kernel took
+//     31.4 us instead of 30.3 on a 2048-token prompt and 28.9 instead of 27.2 on 333
+//     queries over a wrapped ring of 2048 (Qwen2.5-1.5B, Llama-3.2-3B heads). What bounds
+//     it: MFMA, softmax VALU and LDS reads each take about 2000 of the 4500 clocks of a
+//     step (64 keys of the two waves of a SIMD), and the two waves overlap them in part;
+//     then the piece's start (the walk over the blocks, the first tiles' latency) and merge.
 //     Tiles that a wave cannot see are skipped; masks are applied only on the
 //     tiles that cross the causal diagonal or the window start.
 //     Causal work grows with the position, so a query block's key steps may be cut
@@ -101,6 +109,14 @@ __device__ __forceinline__ float ld_dev(const float *p) {
                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
+// max of lanes l and l ^ 32 by a half-wave swap: a lane shuffle would go through LDS, whose
+// results return in order, behind the K and V fragments being read ahead.
+__device__ __forceinline__ float half_max(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
 // f16(v * s) for four values: the f32 product, then its f16 rounding. Kept from fusing
 // into one rounding (v_fma_mix), so that every path storing an output row or a piece's
 // record rounds the same way.
@@ -167,58 +183,76 @@ Window window_of(const AttnArgs &a) {
 // ---------------------------------------------------------------------------
 // 1. Q8_0 window -> f16 K [kvh][pos][HD] and V^T [kvh][HD][pos]
 // ---------------------------------------------------------------------------
-// One wave per 16 window positions of one KV head (a 16-key group of the V^T chunk order).
+// One workgroup per 16 window positions of one KV head (a 16-key group of the V^T chunk
+// order). A head's row of a position is HD/32 blocks of 34 bytes, 4-byte aligned as a
+// whole: the 16 rows of K and V come in through LDS as dwords, five loads a thread, all in
+// flight at once (one wave reading each block's 2-byte words took 34 loads a lane), and
+// leave as 16-byte chunks. 2333 positions x 8 heads of 128: 11.2 -> 10.0 us (64 positions
+// per workgroup, for whole lines of V^T: 12.2).
 constexpr int kWinKeys = 16;
 template <int HD>
-__global__ __launch_bounds__(64) void kv_window_kernel(AttnArgs a, long wlo, int wlen, int wpad, int jb0) {
-  constexpr int NB = HD / 32;
-  __shared__ _Float16 vt[kWinKeys][HD + 2];
+__global__ __launch_bounds__(256) void kv_window_kernel(AttnArgs a, long wlo, int wlen, int wpad, int jb0) {
+  constexpr int NB = HD / 32, ROW = NB * 34, RW = ROW / 4;  // bytes and dwords of a head's row
+  constexpr int WORDS = 2 * kWinKeys * RW, NL = (WORDS + 255) / 256;
+  static_assert(ROW % 4 == 0, "rows of whole dwords");
+  __shared__ uint32_t raw[WORDS];  // K rows, then V rows
   const int kvh = blockIdx.y, j0 = (jb0 + (int)blockIdx.x) * kWinKeys;
   const int cap = a.capacity;
-  const size_t bpp = (size_t)a.n_head_kv * NB * 34;
-  const size_t hoff = (size_t)kvh * NB * 34;
+  const size_t bpp = (size_t)a.n_head_kv * ROW, hoff = (size_t)kvh * ROW;
   _Float16 *kwin = reinterpret_cast<_Float16 *>(a.window);
   _Float16 *vwin = kwin + (size_t)a.n_head_kv * wpad * HD;
-
-  for (int job = threadIdx.x; job < kWinKeys * NB; job += blockDim.x) {
-    const int jj = job / NB, b = job % NB;
+  const int slot0 = (int)((wlo + j0) % cap);
+  uint32_t v[NL];
+#pragma unroll
+  for (int l = 0; l < NL; l++) {
+    const int i = threadIdx.x + 256 * l;
+    const int which = i / (kWinKeys * RW), r = i - which * (kWinKeys * RW);
+    const int jj = r / RW, w = r - jj * RW;
     const int j = j0 + jj;
-    const long p = wlo + j;
-    float dk = 0.0f, dv = 0.0f;
-    const uint16_t *bk = nullptr, *bv = nullptr;
-    if (j < wlen) {
-      const bool staged = p >= a.new_pos0;
-      const size_t off = staged ? (size_t)(p - a.new_pos0) * bpp : (size_t)(p % cap) * bpp;
-      bk = reinterpret_cast<const uint16_t *>((staged ? a.new_k : a.k_ring) + off + hoff + (size_t)b * 34);
-      bv = reinterpret_cast<const uint16_t *>((staged ? a.new_v : a.v_ring) + off + hoff + (size_t)b * 34);
-      dk = (float)__builtin_bit_cast(_Float16, bk[0]);
-      dv = (float)__builtin_bit_cast(_Float16, bv[0]);
-    }
-    _Float16 *kdst = kwin + ((size_t)kvh * wpad + j) * HD + 32 * b;
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      half8 kv8, vv8;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint16_t wk = bk ? bk[1 + 4 * c + e] : 0, wv = bv ? bv[1 + 4 * c + e] : 0;
-        kv8[2 * e] = (_Float16)((float)(int8_t)(wk & 0xff) * dk);
-        kv8[2 * e + 1] = (_Float16)((float)(int8_t)(wk >> 8) * dk);
-        vv8[2 * e] = (_Float16)((float)(int8_t)(wv & 0xff) * dv);
-        vv8[2 * e + 1] = (_Float16)((float)(int8_t)(wv >> 8) * dv);
+    v[l] = 0;  // positions past the window: code 0, scale 0
+    if (i < WORDS && j < wlen) {
+      const long p = wlo + j;
+      const uint8_t *src;
+      if (p >= a.new_pos0) {
+        src = (which ? a.new_v : a.new_k) + (size_t)(p - a.new_pos0) * bpp;
+      } else {
+        int slot = slot0 + jj;
+        while (slot >= cap) slot -= cap;
+        src = (which ? a.v_ring : a.k_ring) + (size_t)slot * bpp;
       }
-      *reinterpret_cast<half8 *>(kdst + 8 * c) = kv8;
-#pragma unroll
-      for (int e = 0; e < 8; e++) vt[jj][32 * b + 8 * c + e] = vv8[e];
+      v[l] = *reinterpret_cast<const uint32_t *>(src + hoff + 4 * w);
     }
   }
-  __syncthreads();
-  // V^T rows: chunk c (8 keys) of row h holds keys 16*(c/2) + kperm(8*(c%2) + e)
-  for (int job = threadIdx.x; job < HD * (kWinKeys / 8); job += blockDim.x) {
-    const int h = job / (kWinKeys / 8), c = job % (kWinKeys / 8);
-    half8 v;
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = vt[16 * (c >> 1) + kperm(8 * (c & 1) + e)][h];
-    *reinterpret_cast<half8 *>(vwin + ((size_t)kvh * HD + h) * (wpad + kVPad) + j0 + 8 * c) = v;
+  for (int l = 0; l < NL; l++)
+    if (threadIdx.x + 256 * l < WORDS) raw[threadIdx.x + 256 * l] = v[l];
+  __syncthreads();
+  // f16(code * d) of element h of row jj
+  const uint8_t *rows = reinterpret_cast<const uint8_t *>(raw);
+  auto scale = [&](const uint8_t *row, int b) { return (float)*reinterpret_cast<const _Float16 *>(row + 34 * b); };
+  for (int c = threadIdx.x; c < kWinKeys * (HD / 8); c += 256) {
+    const int jj = c / (HD / 8), ch = c % (HD / 8);
+    const uint8_t *row = rows + jj * ROW;
+    const float d = scale(row, ch / 4);
+    const uint16_t *codes = reinterpret_cast<const uint16_t *>(row + 34 * (ch / 4) + 2 + 8 * (ch % 4));
+    half8 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      o[2 * e] = (_Float16)((float)(int8_t)(codes[e] & 0xff) * d);
+      o[2 * e + 1] = (_Float16)((float)(int8_t)(codes[e] >> 8) * d);
+    }
+    *reinterpret_cast<half8 *>(kwin + ((size_t)kvh * wpad + j0 + jj) * HD + 8 * ch) = o;
+  }
+  // V^T rows: chunk c (8 keys) of row h holds keys 16*(c/2) + kperm(8*(c%2) + e)
+  for (int job = threadIdx.x; job < HD * (kWinKeys / 8); job += 256) {
+    const int h = job / (kWinKeys / 8), c = job % (kWinKeys / 8);
+    half8 o;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint8_t *row = rows + (kWinKeys + kperm(8 * c + e)) * ROW;
+      o[e] = (_Float16)((float)(int8_t)row[34 * (h / 32) + 2 + h % 32] * scale(row, h / 32));
+    }
+    *reinterpret_cast<half8 *>(vwin + ((size_t)kvh * HD + h) * (wpad + kVPad) + j0 + 8 * c) = o;
   }
 }
 
@@ -330,11 +364,14 @@ __global__ __launch_bounds__(256 * H2, 2 / H2) void flash_attn_kernel(AttnArgs a
     const int ch = (lane % 8) ^ ((hr >> 1) & 7);
     voff[i] = (uint32_t)(hr * vst + 8 * ch) * 2u;
   }
-  // always issued (an idle half reloads a valid tile), so every wave waits the same way
-  auto issue = [&](char *sk, char *sv, int tile) __attribute__((always_inline)) {
+  // a tile past the range reloads the last valid one
+  auto issue_k = [&](char *sk, int tile) __attribute__((always_inline)) {
     const int kb = min(tile, tile1) * kKT;
 #pragma unroll
     for (int i = 0; i < NKI; i++) dma16(rk, sk + RPI * (NKI * qw + i) * KROW, koff[i], kb * HD * 2);
+  };
+  auto issue_v = [&](char *sv, int tile) __attribute__((always_inline)) {
+    const int kb = min(tile, tile1) * kKT;
 #pragma unroll
     for (int i = 0; i < NVI; i++) dma16(rv, sv + 8 * (NVI * qw + i) * kKT * 2, voff[i], kb * 2);
   };
@@ -344,45 +381,37 @@ __global__ __launch_bounds__(256 * H2, 2 / H2) void flash_attn_kernel(AttnArgs a
   for (int i = 0; i < OT; i++) o[i] = floatx16{};
   float mrun = -INFINITY, lrun = 0.0f;
 
-  // --- one tile of 64 keys, as two 32-key online-softmax steps, software-pipelined so
-  // that the MFMAs of one step run under the VALU softmax of the other:
-  //   S0 | S1 + softmax0 | PV0 + softmax1 | PV1
-  auto s_step = [&](const char *sk, int kt, floatx16 &st) __attribute__((always_inline)) {
-    st = floatx16{};
+  // --- MFMAs of one 32-key half tile: S^T of it (one chain of KS), and the PV product of
+  // one (2 OT = KS, OT independent accumulators) ---
+  auto s_mfma = [&](const char *sk, int kt, int s, floatx16 &st) __attribute__((always_inline)) {
     const int row = 32 * kt + l32;
+    const int pos = (2 * s + lg) ^ (row % KCH);
+    const half8 kf = *reinterpret_cast<const half8 *>(sk + row * KROW + 16 * pos);
+    st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], st, 0, 0, 0);
+  };
+  auto pv_mfma = [&](const char *sv, int kt, int s, const half8 (&pp)[2]) __attribute__((always_inline)) {
+    const int jh = s / OT, i = s % OT;
+    const int hr = 32 * i + l32;
+    const int pos = (2 * (2 * kt + jh) + lg) ^ ((hr >> 1) & 7);
+    const half8 vf = *reinterpret_cast<const half8 *>(sv + hr * (kKT * 2) + 16 * pos);
+    o[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pp[jh], o[i], 0, 0, 0);
+  };
+  static_assert(2 * OT == KS, "a half tile's S and PV take equally many MFMAs");
+  // keys outside a query's range (diagonal / window-start tiles only); p_reg0: absolute
+  // position of the lane's register 0
+  auto mask = [&](floatx16 &st, int p_reg0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < KS; s++) {
-      const int pos = (2 * s + lg) ^ (row % KCH);
-      const half8 kf = *reinterpret_cast<const half8 *>(sk + row * KROW + 16 * pos);
-      st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], st, 0, 0, 0);
+    for (int r = 0; r < 16; r++) {
+      const int p = p_reg0 + 8 * (r >> 2) + (r & 3);
+      st[r] = (p > P || p <= P - cap) ? -INFINITY : st[r];
     }
   };
-  auto pv_step = [&](const char *sv, int kt, const half8 (&pbk)[2]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int jh = 0; jh < 2; jh++) {
-      const int j = 2 * kt + jh;  // 16-key step of the tile
-#pragma unroll
-      for (int i = 0; i < OT; i++) {
-        const int hr = 32 * i + l32;
-        const int pos = (2 * j + lg) ^ ((hr >> 1) & 7);
-        const half8 vf = *reinterpret_cast<const half8 *>(sv + hr * (kKT * 2) + 16 * pos);
-        o[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pbk[jh], o[i], 0, 0, 0);
-      }
-    }
-  };
-  // mask (diagonal / window-start tiles only), running max, exp2, sum, P^T as f16
-  auto softmax = [&](floatx16 &st, int p_reg0, bool masked, half8 (&pbk)[2]) __attribute__((always_inline)) -> float {
-    if (masked) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int p = p_reg0 + 8 * (r >> 2) + (r & 3);
-        st[r] = (p > P || p <= P - cap) ? -INFINITY : st[r];
-      }
-    }
+  // running max, exp2, sum, P^T as f16
+  auto softmax = [&](const floatx16 &st, half8 (&pbk)[2]) __attribute__((always_inline)) -> float {
     float mt = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; r++) mt = fmaxf(mt, st[r]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = half_max(mt);
     // The running max only moves when the tile's max exceeds it by more than 2^8 (log2
     // units): P = exp2(s c - m) then stays <= 256, exact to f16 precision, and O and l
     // are rescaled on few tiles. Softmax is shift-invariant, so the result is the same.
@@ -412,66 +441,93 @@ __global__ __launch_bounds__(256 * H2, 2 / H2) void flash_attn_kernel(AttnArgs a
       for (int i = 0; i < OT; i++) o[i] *= alpha;
     }
   };
-  // MFMA / VALU / LDS-read interleave of one pipelined phase (8 MFMAs)
-  auto interleave = [&]() __attribute__((always_inline)) {
+  constexpr int kAhead = 4;  // LDS reads ahead of their MFMA
+  // One phase of the pipeline: the S^T MFMAs of half tile h+1 and the PV MFMAs of h-1 run
+  // under the softmax of h, none of the three waiting for another.
+  auto phase = [&](const char *sk, int kt, floatx16 &snext, const char *sv, int vt, const half8 (&pp)[2],
+                   const floatx16 &scur, half8 (&pc)[2]) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    snext = floatx16{};
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
+    for (int s = 0; s < KS; s++) {
+      s_mfma(sk, kt, s, snext);
+      pv_mfma(sv, vt, s, pp);
+    }
+    const float alpha = softmax(scur, pc);
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+    for (int k = 0; k < 2 * KS; k++) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // 6 VALU
+      if (k + kAhead < 2 * KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
+      __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // 5 VALU
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    rescale(alpha);
+  };
+  // --- the piece's tiles. K runs one tile ahead of V: iteration t takes S^T of tile t+1
+  // and PV of tile t. At its start sb holds S^T of tile t's second half, pa P of its first.
+  floatx16 sa_, sb_;
+  half8 pa[2], pb_[2];
+  auto tile_p0 = [&](int tile) { return (int)wlo + tile * kKT; };  // position of the tile's first key
+  auto visible = [&](int tile) {
+    return tile <= te && wave_live && tile_p0(tile) <= Pw_max && tile_p0(tile) + kKT - 1 > Pw_min - cap;
+  };
+  auto unmasked = [&](int tile) { return tile_p0(tile) + kKT - 1 <= Pw_min && tile_p0(tile) > Pw_max - cap; };
+  auto first = [&](const char *sk, int tile) __attribute__((always_inline)) {  // S^T of both halves, P of the first
+    sa_ = floatx16{};
+    sb_ = floatx16{};
+#pragma unroll
+    for (int s = 0; s < KS; s++) s_mfma(sk, 0, s, sa_);
+#pragma unroll
+    for (int s = 0; s < KS; s++) s_mfma(sk, 1, s, sb_);
+    if (!unmasked(tile)) mask(sa_, tile_p0(tile) + 4 * lg);
+    rescale(softmax(sa_, pa));
+  };
+  auto last = [&](const char *sv, int tile) __attribute__((always_inline)) {  // PV of both halves
+#pragma unroll
+    for (int s = 0; s < KS; s++) pv_mfma(sv, 0, s, pa);
+    if (!unmasked(tile)) mask(sb_, tile_p0(tile) + 32 + 4 * lg);
+    rescale(softmax(sb_, pb_));
+#pragma unroll
+    for (int s = 0; s < KS; s++) pv_mfma(sv, 1, s, pb_);
+  };
+  auto both = [&](const char *sk, const char *sv, int tile) __attribute__((always_inline)) {
+    const int p1 = tile_p0(tile) + 32 + 4 * lg;
+    if (!unmasked(tile)) mask(sb_, p1);
+    phase(sk, 0, sa_, sv, 0, pa, sb_, pb_);
+    if (!unmasked(tile + 1)) mask(sa_, p1 + 32);
+    phase(sk, 1, sb_, sv, 1, pb_, sa_, pa);
+  };
+  // Per iteration: wait for K of tile t+1 and V of tile t, barrier (they landed for all
+  // waves, and every wave finished the previous iteration), prefetch K of t+2 and V of t+1
+  // into the slots the previous iteration read, compute. Both halves of the workgroup run
+  // the same number of iterations and barriers.
+  auto iter = [&](char *k_use, char *k_next, char *v_use, char *v_next, int t) __attribute__((always_inline)) {
+    wait_vmcnt0();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 2 < psteps) issue_k(k_next, tb + t + 2);
+    if (t + 1 < psteps) issue_v(v_next, tb + t + 1);
+    const int tile = tb + t;
+    const bool more = t + 1 < psteps && visible(tile + 1);
+    if (visible(tile) && more) {
+      both(k_use, v_use, tile);
+    } else {
+      if (visible(tile)) last(v_use, tile);
+      if (more) first(k_use, tile + 1);
     }
   };
-  auto compute = [&](const char *sk, const char *sv, int tile, auto kMasked) __attribute__((always_inline)) {
-    constexpr bool M = decltype(kMasked)::value;
-    const int p0 = (int)wlo + tile * kKT;  // absolute position of the tile's first key
-    floatx16 st0, st1;
-    half8 pa[2], pbv[2];
-    s_step(sk, 0, st0);
-    __builtin_amdgcn_sched_barrier(0);
-    s_step(sk, 1, st1);
-    const float al0 = softmax(st0, p0 + 4 * lg, M, pa);
-    interleave();
-    __builtin_amdgcn_sched_barrier(0);
-    rescale(al0);
-    __builtin_amdgcn_sched_barrier(0);
-    pv_step(sv, 0, pa);
-    const float al1 = softmax(st1, p0 + 32 + 4 * lg, M, pbv);
-    interleave();
-    __builtin_amdgcn_sched_barrier(0);
-    rescale(al1);
-    __builtin_amdgcn_sched_barrier(0);
-    pv_step(sv, 1, pbv);
-  };
-  auto tile_work = [&](const char *sk, const char *sv, int tile) __attribute__((always_inline)) {
-    const int p0 = (int)wlo + tile * kKT;
-    if (tile > te || !wave_live || p0 > Pw_max || p0 + kKT - 1 <= Pw_min - cap) return;  // nothing visible
-    if (p0 + kKT - 1 <= Pw_min && p0 > Pw_max - cap) compute(sk, sv, tile, std::false_type{});
-    else compute(sk, sv, tile, std::true_type{});
-  };
-
-  // Per step: wait for this half's tile, barrier (it landed for all waves, and every
-  // wave finished the previous step), prefetch the next tile into the other slot,
-  // compute. Both halves run the same number of steps and barriers.
   auto run = [&](char *k0, char *v0, char *k1, char *v1) __attribute__((always_inline)) {
-    issue(k0, v0, tb);
-    int s = 0;
-    for (; s + 1 < psteps; s += 2) {
-      wait_vmcnt0();
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(k1, v1, tb + s + 1);
-      tile_work(k0, v0, tb + s);
-      wait_vmcnt0();
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(k0, v0, tb + s + 2);
-      tile_work(k1, v1, tb + s + 1);
-    }
-    if (s < psteps) {
-      wait_vmcnt0();
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      tile_work(k0, v0, tb + s);
+    issue_k(k0, tb);
+    issue_v(v0, tb);
+    issue_k(k1, tb + 1);
+    wait_vmcnt<NVI + NKI>();  // K of the first tile
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (psteps > 0 && visible(tb)) first(k0, tb);
+    for (int t = 0; t < psteps; t += 2) {
+      iter(k1, k0, v0, v1, t);
+      if (t + 1 < psteps) iter(k0, k1, v1, v0, t + 1);
     }
   };
   if constexpr (H2 == 1) run(ka0, va0, ka1, va1);
@@ -789,7 +845,7 @@ int32_t launch_hd(const AttnArgs &a, hipStream_t s) {
   // new positions rewrites them with the same values
   auto window_blocks = [&](int b0, int b1) -> int32_t {
     if (b1 <= b0) return SULIMO_HIP_OK;
-    hipLaunchKernelGGL((kv_window_kernel<HD>), dim3(b1 - b0, a.n_head_kv), dim3(64), 0, s, a, w.lo, w.len, w.pad, b0);
+    hipLaunchKernelGGL((kv_window_kernel<HD>), dim3(b1 - b0, a.n_head_kv), dim3(256), 0, s, a, w.lo, w.len, w.pad, b0);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? SULIMO_HIP_OK : hip_fail(e, "kv_window_kernel launch");
   };
