@@ -36,12 +36,11 @@ struct ParkSlot {
   uint64_t posted = 0;
 };
 
-// A ubatch's launches captured once and replayed: two executable graphs split at the
-// wake-up gate (the host records near_event between them), keyed by every value the
+// The middle of a ubatch's launches captured once and replayed, keyed by every value the
 // launches were built from.
 struct PrefillGraph {
   std::vector<uint64_t> key;
-  hipGraphExec_t pre = nullptr, post = nullptr;
+  hipGraphExec_t exec = nullptr;
   uint64_t last_use = 0;
 };
 

@@ -225,8 +225,7 @@ static int32_t create_ctx(int device, bool shared, sulimo_hip_ctx **out) {
 
 void drop_prefill_graphs(sulimo_hip_ctx *ctx) {
   for (PrefillGraph &g : ctx->graphs) {
-    if (g.pre) hipGraphExecDestroy(g.pre);
-    if (g.post) hipGraphExecDestroy(g.post);
+    if (g.exec) hipGraphExecDestroy(g.exec);
   }
   ctx->graphs.clear();
 }
