@@ -1084,11 +1084,15 @@ __global__ __launch_bounds__(256) void split_reduce_norm_kernel(GemmArgs a) {
 // in f32 (exact f16 q-8 products, v_dot2_f32_f16, against x held in LDS) before one
 // multiply by the block's d; the two half-waves of a row combine at the end. x beyond
 // K is zero in LDS, so the odd-block half stage adds nothing.
-constexpr int kGemvMaxXBytes = 64 * 1024;
+// A narrow matrix leaves most CUs idle while each wave walks its row of stages, one memory
+// round trip per U of them: a.splits waves of the workgroup then share a panel's stages
+// (a.split_stages each) and add their sums through LDS, in stage order.
+constexpr int kGemvMaxXBytes = 64 * 1024, kGemvMaxSplits = 16;
 
-template <int MT, int EPI>
-__global__ __launch_bounds__(256) void gemv_q4_kernel(GemmArgs a) {
+template <int MT, int EPI, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kGemvMaxSplits : 256) void gemv_q4_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) _Float16 xs[];  // [MT][kpad]
+  __shared__ float red[SPLIT ? kGemvMaxSplits : 1][MT][32];
   constexpr int U = 8;  // stages in flight per wave
   const int nb = a.k >> 5, nst = (nb + 1) >> 1, kpad = nst * 64;
   for (int i = threadIdx.x; i < MT * kpad / 8; i += blockDim.x) {
@@ -1099,31 +1103,40 @@ __global__ __launch_bounds__(256) void gemv_q4_kernel(GemmArgs a) {
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  int p = blockIdx.x * 4 + (threadIdx.x >> 6);  // panel across the segments
+  int wave = threadIdx.x >> 6, part = 0;
+  int p = blockIdx.x * 4 + wave;  // panel across the segments
+  if constexpr (SPLIT) {
+    wave = __builtin_amdgcn_readfirstlane(wave);
+    part = wave % a.splits;
+    p = blockIdx.x * (blockDim.x / 64 / a.splits) + wave / a.splits;
+  }
   int si = 0;
   for (; si < a.nseg; si++) {
     const int np = (a.seg[si].n + 31) / 32;
     if (p < np) break;
     p -= np;
   }
-  if (si >= a.nseg) return;  // whole waves past the last panel (no barrier below)
-  const GemmSegment seg = a.seg[si];
+  const bool live = si < a.nseg;
+  if (!SPLIT && !live) return;  // (with SPLIT a wave past the last panel keeps the barrier)
+  const GemmSegment seg = a.seg[live ? si : 0];
+  const int sbeg = SPLIT ? part * a.split_stages : 0;
+  const int send = !SPLIT ? nst : live ? min(nst, sbeg + a.split_stages) : 0;
   const uint8_t *rec0 = seg.panels + (size_t)p * nst * kQ4PanelRecord;
   float acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; t++) acc[t] = 0.0f;
-  for (int s0 = 0; s0 < nst; s0 += U) {
+  for (int s0 = sbeg; s0 < send; s0 += U) {
     uint4 qv[U];
     uint32_t sw[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int st = min(s0 + u, nst - 1);  // repeats the last stage, not used below
+      const int st = min(s0 + u, send - 1);  // repeats the last stage, not used below
       qv[u] = *reinterpret_cast<const uint4 *>(rec0 + (size_t)st * kQ4PanelRecord + 16 * lane);
       sw[u] = *reinterpret_cast<const uint32_t *>(rec0 + (size_t)st * kQ4PanelRecord + 1024 + 4 * r);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      if (s0 + u >= nst) break;
+      if (s0 + u >= send) break;
       const int kb = (s0 + u) * 64;
 #pragma unroll
       for (int b = 0; b < 2; b++) {
@@ -1153,8 +1166,21 @@ __global__ __launch_bounds__(256) void gemv_q4_kernel(GemmArgs a) {
   }
   const int row = p * 32 + r;
 #pragma unroll
+  for (int t = 0; t < MT; t++) acc[t] += __shfl_xor(acc[t], 32, 64);
+  if constexpr (SPLIT) {
+    if (!h) {
+#pragma unroll
+      for (int t = 0; t < MT; t++) red[wave][t][r] = acc[t];
+    }
+    __syncthreads();
+    if (part || !live) return;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+      for (int w = 1; w < a.splits; w++) acc[t] += red[wave + w][t][r];
+  }
+#pragma unroll
   for (int t = 0; t < MT; t++) {
-    float v = acc[t] + __shfl_xor(acc[t], 32, 64);
+    float v = acc[t];
     if (h || t >= a.m || row >= seg.n) continue;
     if (seg.bias) v += seg.bias[row];
     const size_t o = (size_t)t * seg.ldo + seg.col0 + row;
@@ -1168,16 +1194,29 @@ __global__ __launch_bounds__(256) void gemv_q4_kernel(GemmArgs a) {
 }
 
 template <int MT>
-int32_t launch_gemv_mt(const GemmArgs &a, hipStream_t s, LaunchStamp st) {
+int32_t launch_gemv_mt(const GemmArgs &args, hipStream_t s, LaunchStamp st) {
+  GemmArgs a = args;
   int panels = 0;
   for (int i = 0; i < a.nseg; i++) panels += (a.seg[i].n + 31) / 32;
+  // waves per panel: enough for eight waves per CU, at least two stages each (1536 x 8960
+  // at one token 37.6 -> 8.7 us, 8960 x 1536 8.7 -> 5.6); a wide matrix fills the CUs as it is
+  const int nst = (a.k / 32 + 1) / 2;
+  a.splits = 1;
+  while (a.splits < kGemvMaxSplits && panels * a.splits < 8 * device_cu_count() && nst >= 4 * a.splits) a.splits *= 2;
+  a.split_stages = (nst + a.splits - 1) / a.splits;
+  const int waves = std::max(4, a.splits);
   const int kpad = ((a.k / 32 + 1) / 2) * 64;
   const size_t lds = (size_t)MT * kpad * 2;
-  const dim3 grid((unsigned)((panels + 3) / 4)), block(256);
+  const int per = waves / a.splits;  // panels per workgroup
+  const dim3 grid((unsigned)((panels + per - 1) / per)), block(64 * waves);
+  auto go = [&](auto split, auto whole) {
+    if (a.splits > 1) launch_stamped(split, grid, block, lds, s, st.start, st.stop, a);
+    else launch_stamped(whole, grid, block, lds, s, st.start, st.stop, a);
+  };
   switch (a.epi) {
-    case EPI_F16: launch_stamped(gemv_q4_kernel<MT, EPI_F16>, grid, block, lds, s, st.start, st.stop, a); break;
-    case EPI_F32: launch_stamped(gemv_q4_kernel<MT, EPI_F32>, grid, block, lds, s, st.start, st.stop, a); break;
-    default: launch_stamped(gemv_q4_kernel<MT, EPI_RESID>, grid, block, lds, s, st.start, st.stop, a); break;
+    case EPI_F16: go(gemv_q4_kernel<MT, EPI_F16, true>, gemv_q4_kernel<MT, EPI_F16, false>); break;
+    case EPI_F32: go(gemv_q4_kernel<MT, EPI_F32, true>, gemv_q4_kernel<MT, EPI_F32, false>); break;
+    default: go(gemv_q4_kernel<MT, EPI_RESID, true>, gemv_q4_kernel<MT, EPI_RESID, false>); break;
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SULIMO_HIP_OK : hip_fail(e, "gemv_q4_kernel launch");

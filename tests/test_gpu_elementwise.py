@@ -6,6 +6,8 @@ import pytest
 
 import oracle
 from sulimo_amd import hip
+from sulimo_amd import synthetic as S
+from tests.test_gpu_gemm import f16_weight_bound, run_gemm
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +51,16 @@ def test_rope_partial_heads_and_widths(ctx, mode, heads, hd, rd, n):
     want[:, :, i0] = x[:, :, i0] * tab[..., 0] - x[:, :, i1] * tab[..., 1]
     want[:, :, i1] = x[:, :, i0] * tab[..., 1] + x[:, :, i1] * tab[..., 0]
     assert np.array_equal(vb.download(np.float16, v.shape).view(np.uint16), want.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("k,m_out", [(8000, 40), (160, 1000), (1536, 9000)])
+def test_gemv_split_stages(ctx, M, k, m_out):
+    """Up to 4 tokens of a narrow matrix: the waves that share a panel's stages (16 of them,
+    2 with one stage left over, and 8 with panels past the last) against the f16-weight bound."""
+    rng = np.random.default_rng(M + k + m_out)
+    w = S.random_q4(rng, m_out, k)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    y = run_gemm(ctx, w.scales, w.quants, x, m_out, k, M)
+    ref = oracle.gemm_q4_0_f16_scalar_reference(w.scales, w.quants, x, m_out, k, M)
+    assert np.all(np.abs(y.astype(np.float64) - ref) <= f16_weight_bound(x, w.scales, w.quants, ref))
