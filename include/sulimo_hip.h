@@ -374,14 +374,16 @@ int32_t sulimo_hip_set_profiling(sulimo_hip_ctx *ctx, int32_t enable);
 
 /* Graph replay of execute_prefill_ubatch (no counterpart in the reference; on by
  * default). The first call with a given set of shapes, buffers and kept-window state
- * captures the launches between the first layer and the last down projection into a HIP
- * graph; later identical calls replay it, which costs the engine thread a few
+ * captures its launches into two HIP graphs, split where the wake-up of the final wait
+ * is gated; later identical calls replay them, which costs the engine thread a few
  * microseconds of CPU instead of one launch each (the reference's engine thread must
- * stay under 5 % of a core while the GPU runs a prefill). The dozen launches before and
- * after it, models of fewer than 4 layers, and calls with profiling on or with
- * per-position outputs run eagerly. Results are bit-identical either way.
+ * stay under 5 % of a core while the GPU runs a prefill). Calls with profiling on or
+ * with per-position outputs run eagerly. Results are bit-identical either way.
  * Disabling it also frees the cached graphs. */
 int32_t sulimo_hip_set_graph_replay(sulimo_hip_ctx *ctx, int32_t enable);
+/* How many prefill calls of the context captured their launches, and how many replayed
+ * launches that an earlier call had captured. */
+int32_t sulimo_hip_get_graph_replay_counts(const sulimo_hip_ctx *ctx, uint64_t *captured, uint64_t *replayed);
 /* Backend tuning switch (no counterpart in the reference). When the attention splits a
  * query block's keys over several workgroups, the last workgroup to finish a block
  * merges its pieces (default), or with enable != 0 a separate kernel launch merges them.

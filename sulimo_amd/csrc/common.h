@@ -36,11 +36,12 @@ struct ParkSlot {
   uint64_t posted = 0;
 };
 
-// The middle of a ubatch's launches captured once and replayed, keyed by every value the
+// A ubatch's launches captured once and replayed: two executable graphs split at the
+// wake-up gate (the host records near_event between them), keyed by every value the
 // launches were built from.
 struct PrefillGraph {
   std::vector<uint64_t> key;
-  hipGraphExec_t exec = nullptr;
+  hipGraphExec_t pre = nullptr, post = nullptr;
   uint64_t last_use = 0;
 };
 
@@ -84,6 +85,7 @@ struct sulimo_hip_ctx {
   bool attn_merge_kernel = false;
   std::vector<PrefillGraph> graphs;
   uint64_t graph_tick = 0;
+  uint64_t graph_captures = 0, graph_replays = 0;
 };
 
 // GEMM-layout copy of one Q4_0 matrix (or an interleaved gate/up pair), built from

@@ -668,24 +668,22 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
     return rc;
   const bool want_outputs = outputs && (outputs->logits_all || outputs->argmax_all || outputs->unfused);
 
-  float *rope_tab = reinterpret_cast<float *>(ws + off_r);
-  // The launches of the ubatch, in order: start, then front and down of every layer (up to
-  // the gate/up projection; the down projection), then finish.
-  auto start = [&]() -> int32_t {
+  // Every launch of the ubatch, in order. gate() runs where the wake-up of the final
+  // wait is gated (before the last down projection): it records near_event, or, under
+  // graph capture, closes the first graph and opens the second.
+  auto body = [&](auto &&gate) -> int32_t {
   int32_t rc = SULIMO_HIP_OK;
   if ((rc = timed(ctx, PROF_NORM, 0, 6.0 * n * D, [&] { return launch_f16_to_f32(dp<const uint16_t>(scratch->x), xres, n * D, s); }))) return rc;
+  float *rope_tab = reinterpret_cast<float *>(ws + off_r);
   if ((rc = timed(ctx, PROF_ROPE_KV, 0, 8.0 * n * (cfg->rope_dim / 2), [&] {
          return launch_rope_table(rope_tab, cfg->rope_dim, cfg->rope_base, (int)start_pos, in, s);
        })))
     return rc;
-  return SULIMO_HIP_OK;
-  };
   // An EPI_RESID GEMM whose K split runs the RMSNorm of the rows it updates (o-proj:
   // the FFN norm, down-proj: the next layer's attention norm or the output norm) leaves
   // h ready, and the separate norm launch is skipped.
   bool h_ready = false;
-  auto front = [&](size_t l) -> int32_t {
-    int32_t rc = SULIMO_HIP_OK;
+  for (size_t l = 0; l < L; l++) {
     const sulimo_hip_layer_tensors &T = tensors->layers[l];
     uint8_t *ring_k = dp<uint8_t>(kv->k_buffers[l]);
     uint8_t *ring_v = dp<uint8_t>(kv->v_buffers[l]);
@@ -696,7 +694,7 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
                      })))
       return rc;
     const uint8_t *pq = panels[6 * l], *pk = panels[6 * l + 1], *pv = panels[6 * l + 2],
-                  *po = panels[6 * l + 3], *pgu = panels[6 * l + 4];
+                  *po = panels[6 * l + 3], *pgu = panels[6 * l + 4], *pd = panels[6 * l + 5];
     // attention arguments first: the RoPE + Q8_0 store also writes the f16 window
     // entries of the new positions
     AttnArgs at{};
@@ -837,12 +835,7 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
     } else if ((rc = timed_gemm(ctx, PROF_GEMM_GATE_UP, gemm_flop(gu), gemm_bytes(gu),
                                 [&](const LaunchStamp *st) { return launch_gemm_q4_0(gu, s, nullptr, st); })))
       return rc;
-    return SULIMO_HIP_OK;
-  };
-  // 11-12. down projection, residual add fused
-  auto down = [&](size_t l) -> int32_t {
-    int32_t rc = SULIMO_HIP_OK;
-    const uint8_t *pd = panels[6 * l + 5];
+    // 11-12. down projection, residual add fused
     GemmArgs gd{};
     gd.x = dp<const uint16_t>(scratch->ffn_swiglu);
     gd.m = in;
@@ -854,6 +847,8 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
     gd.part = gemm_part;
     gd.part_bytes = gemm_ws;
     const bool last = l + 1 == L;
+    // the wake-up of the final wait is gated here, some 50-100 us before the end
+    if (last && (rc = gate())) return rc;
     gd.norm_w = dp<const float>(last ? tensors->output_norm : tensors->layers[l + 1].attn_norm);
     gd.norm_out = dp<uint16_t>(scratch->h);
     gd.norm_x16 = last ? dp<uint16_t>(scratch->x) : nullptr;
@@ -870,10 +865,7 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
     } else if ((rc = timed_gemm(ctx, PROF_GEMM_DOWN, gemm_flop(gd), gemm_bytes(gd),
                                 [&](const LaunchStamp *st) { return launch_gemm_q4_0(gd, s, &h_ready, st); })))
       return rc;
-    return SULIMO_HIP_OK;
-  };
-  auto finish = [&]() -> int32_t {
-  int32_t rc = SULIMO_HIP_OK;
+  }
   // 13. output RMSNorm of all n rows (h), final residual back to scratch.x as f16
   if (!h_ready && (rc = timed(ctx, PROF_NORM, 0, 8.0 * n * D + 4.0 * D, [&] {
                      return launch_rmsnorm_f32(xres, dp<const float>(tensors->output_norm), dp<uint16_t>(scratch->h),
@@ -904,31 +896,14 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
   return SULIMO_HIP_OK;
   };
 
-  // Graph replay covers the middle of a deep model's ubatch: everything between the first
-  // layer and the last down projection. The dozen launches around it cost the thread 2.5 us
-  // each, and one graph instead of two (one on each side of the gate) is one capture and
-  // one launch less: the first call of a 28-layer model takes 6.7 ms instead of 7.6, a
-  // replay the same (1.60 ms at 23 tokens). Models of fewer layers launch one by one, which
-  // the GPU runs faster than a graph's nodes (one Llama-3.2-3B layer of 4096 tokens 1118 ->
-  // 1073 us; 28 layers of 23 tokens 1604 -> 1492 us, for a third of the thread's time).
-  constexpr size_t kGraphLayers = 4;
-  // The wake-up of the final wait is gated before the last down projection, some 50-100 us
-  // before the end. With per-position outputs the LM head over all rows follows that point,
-  // so the wake-up is not gated (the host function ends the queue).
-  auto gate = [&]() -> int32_t {
-    if (!want_outputs) SULIMO_HIP_TRY(hipEventRecord(ctx->near_event, s));
-    return SULIMO_HIP_OK;
-  };
-  // layers 1 .. L-1 without the last down projection
-  auto middle = [&]() -> int32_t {
-    int32_t rc = SULIMO_HIP_OK;
-    for (size_t l = 1; l < L; l++)
-      if ((rc = front(l)) || (l + 1 < L && (rc = down(l)))) return rc;
-    return SULIMO_HIP_OK;
-  };
-  if ((rc = start()) || (rc = front(0)) || (L > 1 && (rc = down(0)))) return rc;
-  if (!ctx->graph_replay || ctx->prof || want_outputs || L < kGraphLayers) {
-    if ((rc = middle())) return rc;
+  if (!ctx->graph_replay || ctx->prof || want_outputs) {
+    // Eager launches. With per-position outputs the LM head over all rows follows the
+    // gate point, so the wake-up is not gated (the host function ends the queue).
+    rc = body([&]() -> int32_t {
+      if (!want_outputs) SULIMO_HIP_TRY(hipEventRecord(ctx->near_event, s));
+      return SULIMO_HIP_OK;
+    });
+    if (rc) return rc;
   } else {
     // Graph replay: the key holds every value the launches are built from.
     std::vector<uint64_t> key;
@@ -963,32 +938,53 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
     for (PrefillGraph &g : ctx->graphs)
       if (g.key == key) hit = &g;
     if (!hit) {
-      hipGraph_t g = nullptr;
+      hipGraph_t g1 = nullptr, g2 = nullptr;
       SULIMO_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      const int32_t brc = middle();
-      hipError_t ce = hipStreamEndCapture(s, &g);
+      bool split = false;
+      int32_t brc = body([&]() -> int32_t {
+        hipError_t e = hipStreamEndCapture(s, &g1);
+        if (e != hipSuccess) return hip_fail(e, "graph capture");
+        e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+        if (e != hipSuccess) return hip_fail(e, "graph capture");
+        split = true;
+        return SULIMO_HIP_OK;
+      });
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      hipError_t ce = hipStreamIsCapturing(s, &cs);
+      if (ce == hipSuccess && cs != hipStreamCaptureStatusNone) ce = hipStreamEndCapture(s, &g2);
       PrefillGraph pg;
       pg.key = std::move(key);
-      if (brc == SULIMO_HIP_OK && ce == hipSuccess && g) ce = hipGraphInstantiate(&pg.exec, g, nullptr, nullptr, 0);
-      else if (brc == SULIMO_HIP_OK && ce == hipSuccess) ce = hipErrorInvalidValue;
-      if (g) hipGraphDestroy(g);
+      if (brc == SULIMO_HIP_OK && ce == hipSuccess && split && g1 && g2) {
+        ce = hipGraphInstantiate(&pg.pre, g1, nullptr, nullptr, 0);
+        if (ce == hipSuccess) ce = hipGraphInstantiate(&pg.post, g2, nullptr, nullptr, 0);
+      } else if (brc == SULIMO_HIP_OK && ce == hipSuccess) {
+        ce = hipErrorInvalidValue;
+      }
+      if (g1) hipGraphDestroy(g1);
+      if (g2) hipGraphDestroy(g2);
       if (brc || ce != hipSuccess) {
-        if (pg.exec) hipGraphExecDestroy(pg.exec);
+        if (pg.pre) hipGraphExecDestroy(pg.pre);
+        if (pg.post) hipGraphExecDestroy(pg.post);
         return brc ? brc : hip_fail(ce, "prefill graph capture");
       }
       if (ctx->graphs.size() >= 8) {  // evict the least recently used
         auto lru = std::min_element(ctx->graphs.begin(), ctx->graphs.end(),
                                     [](const PrefillGraph &a, const PrefillGraph &b) { return a.last_use < b.last_use; });
-        hipGraphExecDestroy(lru->exec);
+        hipGraphExecDestroy(lru->pre);
+        hipGraphExecDestroy(lru->post);
         ctx->graphs.erase(lru);
       }
       ctx->graphs.push_back(std::move(pg));
       hit = &ctx->graphs.back();
+      ctx->graph_captures++;
+    } else {
+      ctx->graph_replays++;
     }
     hit->last_use = ++ctx->graph_tick;
-    SULIMO_HIP_TRY(hipGraphLaunch(hit->exec, s));
+    SULIMO_HIP_TRY(hipGraphLaunch(hit->pre, s));
+    SULIMO_HIP_TRY(hipEventRecord(ctx->near_event, s));
+    SULIMO_HIP_TRY(hipGraphLaunch(hit->post, s));
   }
-  if ((rc = gate()) || (rc = down(L - 1)) || (rc = finish())) return rc;
   // 15. one wait for the whole ubatch (the thread sleeps while the GPU works)
   rc = wait_parked(ctx, want_outputs ? nullptr : ctx->near_event);
   if (rc == SULIMO_HIP_OK && keep_win) {

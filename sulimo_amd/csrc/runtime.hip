@@ -225,7 +225,8 @@ static int32_t create_ctx(int device, bool shared, sulimo_hip_ctx **out) {
 
 void drop_prefill_graphs(sulimo_hip_ctx *ctx) {
   for (PrefillGraph &g : ctx->graphs) {
-    if (g.exec) hipGraphExecDestroy(g.exec);
+    if (g.pre) hipGraphExecDestroy(g.pre);
+    if (g.post) hipGraphExecDestroy(g.post);
   }
   ctx->graphs.clear();
 }
@@ -370,6 +371,13 @@ int32_t sulimo_hip_set_graph_replay(sulimo_hip_ctx *ctx, int32_t enable) {
   if (rc) return rc;
   ctx->graph_replay = enable != 0;
   if (!ctx->graph_replay) drop_prefill_graphs(ctx);
+  return SULIMO_HIP_OK;
+}
+
+int32_t sulimo_hip_get_graph_replay_counts(const sulimo_hip_ctx *ctx, uint64_t *captured, uint64_t *replayed) {
+  if (!ctx || !captured || !replayed) return fail(SULIMO_HIP_ERR_INVALID_ARGUMENT, "ctx, captured or replayed is null");
+  *captured = ctx->graph_captures;
+  *replayed = ctx->graph_replays;
   return SULIMO_HIP_OK;
 }
 

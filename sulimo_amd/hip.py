@@ -181,6 +181,7 @@ def _declare(L):
         "sulimo_hip_rope_table": (I32, [P, SZ, F, SZ, SZ, P]),
         "sulimo_hip_set_profiling": (I32, [P, I32]),
         "sulimo_hip_set_graph_replay": (I32, [P, I32]),
+        "sulimo_hip_get_graph_replay_counts": (I32, [P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
         "sulimo_hip_set_attention_merge_kernel": (I32, [P, I32]),
         "sulimo_hip_get_prefill_stats": (I32, [P, C.POINTER(PrefillStats)]),
         "sulimo_hip_timer_start": (I32, [P]),
@@ -248,6 +249,12 @@ class HipContext:
 
     def set_graph_replay(self, enable: bool):
         _check(lib().sulimo_hip_set_graph_replay(self.handle, 1 if enable else 0))
+
+    def graph_replay_counts(self) -> tuple[int, int]:
+        """(prefill calls that captured their launches, calls that replayed captured ones)."""
+        cap, rep = C.c_uint64(), C.c_uint64()
+        _check(lib().sulimo_hip_get_graph_replay_counts(self.handle, C.byref(cap), C.byref(rep)))
+        return int(cap.value), int(rep.value)
 
     def set_attention_merge_kernel(self, enable: bool):
         """Merge split attention blocks in a separate kernel (True) or in the last

@@ -215,26 +215,36 @@ def _graph_sequence(ctx, hm, toks, cap, calls, reps):
     return out
 
 
-@pytest.mark.parametrize("calls,cap", [([(0, 512)], 1024),                # prompt from position 0, kept window
-                                       ([(0, 512), (512, 256)], 1024),    # resume over the kept window
-                                       ([(0, 512), (512, 256)], 600)],    # the second ubatch wraps the ring
-                         ids=["fresh", "resume", "wrap"])
-def test_graph_replay_bit_identical(calls, cap):
+@pytest.mark.parametrize("layers,calls,cap", [
+    (2, [(0, 512)], 1024),                # prompt from position 0, kept window
+    (2, [(0, 512), (512, 256)], 1024),    # resume over the kept window
+    (2, [(0, 512), (512, 256)], 600),     # the second ubatch wraps the ring
+    (1, [(0, 40), (40, 1)], 256),         # the first layer is the last
+    (5, [(0, 96), (96, 23), (119, 23), (142, 5)], 1024),  # short turns, each at its own start
+], ids=["fresh", "resume", "wrap", "one_layer", "turns"])
+def test_graph_replay_bit_identical(layers, calls, cap):
     """Graph replay (the default) against eager launches: the same sequence of prefill
     calls, repeated three times with the program's own GEMM and wait between calls, gives
     logits and K/V ring bytes identical to the same sequence run eagerly, after every
-    call (the first repetition captures each call's graphs, the others replay them)."""
-    cfg = dataclasses.replace(S.QWEN25_1_5B, n_layers=2, vocab=4096)
+    call (the first repetition captures each call's graphs, the others replay them; the
+    context's counts show that both happened, whatever the depth of the model)."""
+    cfg = dataclasses.replace(S.QWEN25_1_5B, n_layers=layers, vocab=4096)
     hm = S.make_model(cfg, 70, zero_mean=True)
     toks = S.random_tokens(71, 768, cfg.vocab)
     ctx = hip.HipContext.get_or_init(0)
     try:
         ctx.set_graph_replay(False)
+        before = ctx.graph_replay_counts()
         eager = _graph_sequence(ctx, hm, toks, cap, calls, 3)
+        assert ctx.graph_replay_counts() == before
         ctx.set_graph_replay(True)
         replay = _graph_sequence(ctx, hm, toks, cap, calls, 3)
+        captured, replayed = (b - a for a, b in zip(before, ctx.graph_replay_counts()))
     finally:
         ctx.set_graph_replay(True)
+    # every call captured or replayed; once the workspace has its size (one repetition), all replay
+    assert captured + replayed == 3 * len(calls)
+    assert captured >= len(calls) and replayed >= len(calls)
     for i, (lg, k, v) in enumerate(replay):
         le, ke, ve = eager[i]
         assert np.array_equal(lg.view(np.uint32), le.view(np.uint32)), f"logits of call {i}"
