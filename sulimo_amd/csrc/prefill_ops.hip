@@ -4,6 +4,7 @@
 // kv_store_q8_0 :72-116, silu_mul_f16 :240-253, add_f16 :256-266) and the host
 // embedding gather of crates/sulimo-engine/src/scheduler.rs:329-374.
 #include "common.h"
+#include "rope_route.h"
 
 namespace sulimo {
 namespace {
@@ -142,12 +143,11 @@ __global__ void rope_f16_kernel(_Float16 *vec, int head_count, int head_dim, int
 // every load comes before the first store. More heads per thread would leave too few waves
 // for a short ubatch (64 pairs of 1000 tokens make 16000 threads a head group). 1000 tokens
 // x 12 heads of 128: 8.1 -> 5.3 us.
-constexpr int kRopeHeads = 4;
-__global__ __launch_bounds__(256) void rope_f16_vec_kernel(_Float16 *vec, int head_count, int head_dim, int rope_dim,
+__global__ __launch_bounds__(kRopeThreads) void rope_f16_vec_kernel(_Float16 *vec, int head_count, int head_dim, int rope_dim,
                                                            float base, int mode, int start_pos, int n) {
   typedef _Float16 half4v __attribute__((ext_vector_type(4)));
   const int half = rope_dim / 2, quads = half / 4;
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;  // n * quads fits int (a buffer holds n rows)
+  const int gid = blockIdx.x * blockDim.x + threadIdx.x;  // int holds it (rope_vec_grid)
   if (gid >= n * quads) return;
   const int t = gid / quads, i = (gid - t * quads) * 4;
   const int h0 = blockIdx.y * kRopeHeads;
@@ -585,10 +585,9 @@ int32_t launch_rope_f16(uint16_t *vec, int head_count, int head_dim, int rope_di
                         float freq_base, int mode, int start_pos, int n, hipStream_t s) {
   const size_t total = (size_t)n * head_count * (rope_dim / 2);
   if (total == 0) return SULIMO_HIP_OK;
-  // whole quads of pairs, in rows and halves of 16- and 8-byte alignment
-  if (rope_dim % 8 == 0 && head_dim % 8 == 0) {
-    hipLaunchKernelGGL(rope_f16_vec_kernel, dim3(blocks_for((size_t)n * (rope_dim / 8), 256), (head_count + kRopeHeads - 1) / kRopeHeads), dim3(256), 0,
-                       s, reinterpret_cast<_Float16 *>(vec), head_count, head_dim, rope_dim, freq_base, mode, start_pos, n);
+  if (const RopeVecGrid g = rope_vec_grid(head_count, head_dim, rope_dim, n); g.x) {
+    hipLaunchKernelGGL(rope_f16_vec_kernel, dim3(g.x, g.y), dim3(kRopeThreads), 0, s, reinterpret_cast<_Float16 *>(vec),
+                       head_count, head_dim, rope_dim, freq_base, mode, start_pos, n);
     return check_launch("rope_f16_vec_kernel");
   }
   hipLaunchKernelGGL(rope_f16_kernel, dim3(blocks_for(total, 256)), dim3(256), 0, s,
