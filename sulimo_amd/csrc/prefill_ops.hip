@@ -221,8 +221,8 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const _Float16 *act, uint
 
 // The elementwise kernels move 8 elements per thread with 16-byte accesses (element by
 // element they were bound by the instructions, not the bytes: silu_mul of 9 M elements
-// 16.6 -> 10.7 us, 5.0 TB/s, the rate of a large copy); the last thread takes the odd elements. The arrays start at device
-// allocations (256-byte aligned).
+// 16.6 -> 10.7 us, 5.0 TB/s, the rate of a large copy); the last thread takes the odd
+// elements. The arrays start at device allocations (256-byte aligned).
 __global__ __launch_bounds__(256) void silu_mul_kernel(const _Float16 *g, const _Float16 *u, _Float16 *out, size_t total) {
   const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
   if (i + 8 <= total) {
@@ -232,12 +232,12 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const _Float16 *g, const 
     for (int e = 0; e < 8; e += 2) {
       // f16(t u) in one rounding (v_fma_mix), as the compiler rounds the fused SwiGLU's
       // product, so that both give identical bits; a partly written register is read one
-      // wait state later
+      // wait state later, and w is written before the second pair is read
       const float g0 = (float)a[e], g1 = (float)a[e + 1];
       const float t0 = silu_mul(g0, 1.0f), t1 = silu_mul(g1, 1.0f), u0 = (float)b[e], u1 = (float)b[e + 1];
       uint32_t w = 0;
       asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\ts_nop 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0\n\ts_nop 0"
-          : "+v"(w) : "v"(t0), "v"(u0), "v"(t1), "v"(u1));
+          : "+&v"(w) : "v"(t0), "v"(u0), "v"(t1), "v"(u1));
       o[e / 2] = w;
     }
     *reinterpret_cast<uint4 *>(out + i) = uint4{o[0], o[1], o[2], o[3]};

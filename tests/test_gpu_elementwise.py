@@ -34,6 +34,20 @@ def test_silu_and_add_edges(ctx, total):
     assert np.array_equal(got[total:], g[total:])
 
 
+def test_silu_vector_and_single_elements_agree(ctx):
+    """Bit for bit: 7 elements run one by one, 8 as two registers of packed pairs, each of
+    whose products must read its own operands."""
+    rng = np.random.default_rng(40)
+    for i in range(64):
+        g, u = ((rng.standard_normal(8) * 4.0 ** rng.integers(-3, 3)).astype(np.float16) for _ in range(2))
+        got = []
+        for total in (7, 8):
+            ob = up(ctx, np.zeros(8, np.float16))
+            hip.enqueue_silu_mul(ctx, up(ctx, g), up(ctx, u), ob, total)
+            got.append(ob.download(np.uint16, 8))
+        assert np.array_equal(got[0][:7], got[1][:7]), i
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("heads,hd,rd,n", [(5, 64, 40, 3), (1, 128, 128, 1), (7, 64, 12, 5), (9, 32, 32, 70)])
 def test_rope_partial_heads_and_widths(ctx, mode, heads, hd, rd, n):
