@@ -503,6 +503,7 @@ __global__ __launch_bounds__(256 * H2, 2 / H2) void flash_attn_kernel(AttnArgs a
   // into the slots the previous iteration read, compute. Both halves of the workgroup run
   // the same number of iterations and barriers.
   auto iter = [&](char *k_use, char *k_next, char *v_use, char *v_next, int t) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);  // the MFMAs that wait for the last LDS reads stay above
     wait_vmcnt0();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -518,9 +519,11 @@ __global__ __launch_bounds__(256 * H2, 2 / H2) void flash_attn_kernel(AttnArgs a
     }
   };
   auto run = [&](char *k0, char *v0, char *k1, char *v1) __attribute__((always_inline)) {
-    issue_k(k0, tb);
+    issue_k(k0, tb);  // first: the wait below counts on all others being younger
+    __builtin_amdgcn_sched_barrier(0);
     issue_v(v0, tb);
     issue_k(k1, tb + 1);
+    __builtin_amdgcn_sched_barrier(0);
     wait_vmcnt<NVI + NKI>();  // K of the first tile
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
