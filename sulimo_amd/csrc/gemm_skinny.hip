@@ -59,7 +59,6 @@ struct SkinnyArgs {
   int npairs;       // steps of 128 k
   int split_pairs;  // steps per K split
   int xrows;        // rows of X staged per step (m rounded up to 4)
-  int red_tiles;    // 16-row tiles per round of the sum over the waves
 };
 
 // Output columns of one workgroup.
@@ -254,46 +253,145 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
     }
   }
 
-  // --- the waves' sums meet in LDS (over the X slots): red_tiles 16-row tiles at a time,
-  // all of them where they fit. A tile is 4 NF groups of 16 lanes, group (f, gg) = rows
-  // 4gg .. +3 of fragment f's columns; an owner wave adds 4 groups over the waves, in wave
-  // order, and runs the epilogue for them. ---
+  // --- the waves' sums meet in LDS (over the X slots). A 16-row tile is 4 NF groups of 16
+  // lanes, group (f, gg) = rows 4gg .. +3 of fragment f's columns; an owner wave adds 4
+  // groups over the waves, in wave order, and runs the epilogue for them. ---
   float4 *red = reinterpret_cast<float4 *>(smem);
-  for (int i0 = 0; i0 < MT; i0 += sa.red_tiles) {
-    lds_barrier();
+  lds_barrier();
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-      if (i < i0 || i >= i0 + sa.red_tiles) continue;
+  for (int i = 0; i < MT; i++)
 #pragma unroll
-      for (int f = 0; f < NF; f++)
-        red[(((i - i0) * nwaves + wave) * NF + f) * 64 + lane] = float4{acc[i][f][0], acc[i][f][1], acc[i][f][2], acc[i][f][3]};
-    }
-    lds_barrier();
-    const int groups = NF * min(sa.red_tiles, MT - i0);
-    for (int o = wave; o < groups; o += nwaves) {
-      const int i = i0 + o / NF;  // 16-row tile
-      const int id = 4 * (o % NF) + g, f = id % NF, gg = id / NF;
-      const float4 *red_t = red + (size_t)(o / NF) * nwaves * NF * 64;
-      float4 v = red_t[f * 64 + 16 * gg + r16];
+    for (int f = 0; f < NF; f++)
+      red[((i * nwaves + wave) * NF + f) * 64 + lane] = float4{acc[i][f][0], acc[i][f][1], acc[i][f][2], acc[i][f][3]};
+  lds_barrier();
+  for (int o = wave; o < MT * NF; o += nwaves) {
+    const int i = o / NF;  // 16-row tile
+    const int id = 4 * (o % NF) + g, f = id % NF, gg = id / NF;
+    const float4 *red_t = red + (size_t)i * nwaves * NF * 64;
+    float4 v = red_t[f * 64 + 16 * gg + r16];
 #pragma unroll 4
-      for (int w = 1; w < nwaves; w++) {
-        const float4 t = red_t[(w * NF + f) * 64 + 16 * gg + r16];
-        v.x += t.x;
-        v.y += t.y;
-        v.z += t.z;
-        v.w += t.w;
-      }
-      // the lane's column before the quad transpose, and row / first column after it
-      const int row = 16 * i + 4 * gg + qj;
-      if constexpr (EPI == EPI_SWIGLU) {
-        // gate fragments (lanes 0-31) and up fragments (lanes 32-63), f16-rounded first
-        const float gv[4] = {(float)(_Float16)v.x, (float)(_Float16)v.y, (float)(_Float16)v.z, (float)(_Float16)v.w};
-        float s[4];
+    for (int w = 1; w < nwaves; w++) {
+      const float4 t = red_t[(w * NF + f) * 64 + 16 * gg + r16];
+      v.x += t.x;
+      v.y += t.y;
+      v.z += t.z;
+      v.w += t.w;
+    }
+    // the lane's column before the quad transpose, and row / first column after it
+    const int row = 16 * i + 4 * gg + qj;
+    if constexpr (EPI == EPI_SWIGLU) {
+      // gate fragments (lanes 0-31) and up fragments (lanes 32-63), f16-rounded first
+      const float gv[4] = {(float)(_Float16)v.x, (float)(_Float16)v.y, (float)(_Float16)v.z, (float)(_Float16)v.w};
+      float s[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) s[e] = silu_mul(gv[e], __shfl_xor(gv[e], 32, 64));
-        const uint2 w = quad_t16(pack_h2(s[0], s[1]), pack_h2(s[2], s[3]), qj);
-        const int col = UC * u + 16 * (f & 1) + cq4;
-        if (lane < 32 && row < a.m && col < seg.n) {
+      for (int e = 0; e < 4; e++) s[e] = silu_mul(gv[e], __shfl_xor(gv[e], 32, 64));
+      const uint2 w = quad_t16(pack_h2(s[0], s[1]), pack_h2(s[2], s[3]), qj);
+      const int col = UC * u + 16 * (f & 1) + cq4;
+      if (lane < 32 && row < a.m && col < seg.n) {
+        _Float16 *dst = reinterpret_cast<_Float16 *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col;
+        if (((seg.ldo | seg.col0) & 3) == 0 && ((uintptr_t)seg.out & 7) == 0 && col + 4 <= seg.n) {
+          *reinterpret_cast<uint2 *>(dst) = w;
+        } else {
+          const uint32_t ww[2] = {w.x, w.y};
+          for (int e = 0; e < 4 && col + e < seg.n; e++)
+            reinterpret_cast<uint16_t *>(dst)[e] = (uint16_t)(ww[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    } else if constexpr (EPI == EPI_ROPE) {
+      // RoPE + Q8_0 K/V store: the values and rounding points of gemm_q4_0.hip's RoPE
+      // epilogue. Lanes 0-31 hold 32 columns of the first half of a head, lanes 32-63
+      // the columns head_dim/2 further: a Q8_0 block is half a wave, NeoX partners are
+      // lanes l and l ^ 32.
+      const GemmRope &rp = a.rope;
+      const int hd = rp.head_dim;
+      const bool neox = rp.mode != 0, rotate = si < 2;
+      const int fcol = rope_col(f);  // fragment's first column
+      const float b = seg.bias ? seg.bias[fcol + r16] : 0.0f;
+      const int col = fcol + cq4, e0 = col & (hd - 1);
+      float4 ca = ca0, cb = cb0;
+      if (rotate && o != own0) rope_cs(row, e0, ca, cb);
+      const uint2 xv = quad_t16(pack_h2(v.x + b, v.y + b), pack_h2(v.z + b, v.w + b), qj);
+      const half2v x01 = as_h2(xv.x), x23 = as_h2(xv.y);
+      const float x[4] = {(float)x01[0], (float)x01[1], (float)x23[0], (float)x23[1]};
+      float out[4] = {x[0], x[1], x[2], x[3]};
+      if (rotate && neox) {
+        const half2v p01 = as_h2((uint32_t)__shfl_xor((int)xv.x, 32, 64)), p23 = as_h2((uint32_t)__shfl_xor((int)xv.y, 32, 64));
+        const float p[4] = {(float)p01[0], (float)p01[1], (float)p23[0], (float)p23[1]};
+        const float cc[4] = {ca.x, ca.z, cb.x, cb.z}, ss[4] = {ca.y, ca.w, cb.y, cb.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          out[j] = lane < 32 ? rot_sub(x[j], cc[j], p[j], ss[j]) : rot_add(p[j], ss[j], x[j], cc[j]);
+      } else if (rotate) {
+        const float cc[2] = {ca.x, ca.z}, ss[2] = {ca.y, ca.w};
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+          out[j] = rot_sub(x[j], cc[j / 2], x[j + 1], ss[j / 2]);
+          out[j + 1] = rot_add(x[j], ss[j / 2], x[j + 1], cc[j / 2]);
+        }
+      }
+      const bool ok = row < a.m;
+      if (si == 0) {
+        if (ok)
+          *reinterpret_cast<uint2 *>(reinterpret_cast<_Float16 *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col) =
+              uint2{pack_h2(out[0], out[1]), pack_h2(out[2], out[3])};
+        continue;
+      }
+      float amax = fmaxf(fmaxf(fabsf(out[0]), fabsf(out[1])), fmaxf(fabsf(out[2]), fabsf(out[3])));
+#pragma unroll
+      for (int sh = 4; sh <= 16; sh *= 2) amax = fmaxf(amax, __shfl_xor(amax, sh, 64));
+      const float d = amax / 127.0f;
+      const float id = d != 0.0f ? 1.0f / d : 0.0f;
+      float qc[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) qc[j] = fminf(fmaxf(roundf(out[j] * id), -128.0f), 127.0f);
+      const int kvh = head, e = e0;
+      if (ok) {
+        int slot_i = rp.slot0 + row;
+        if (slot_i >= rp.wrap) slot_i %= rp.wrap;
+        uint8_t *blk = (si == 1 ? rp.k_dst : rp.v_dst) + (size_t)slot_i * rp.row_bytes +
+                       (size_t)(kvh * (hd >> 5) + (e >> 5)) * 34;
+        if ((e & 31) == 0) *reinterpret_cast<_Float16 *>(blk) = (_Float16)d;
+        uint16_t *codes = reinterpret_cast<uint16_t *>(blk + 2 + (e & 31));  // 2-byte aligned
+#pragma unroll
+        for (int j = 0; j < 4; j += 2)
+          codes[j / 2] = (uint16_t)((uint8_t)(int8_t)(int)qc[j] | ((uint16_t)(uint8_t)(int8_t)(int)qc[j + 1] << 8));
+      }
+      if (!rp.win.k) continue;
+      // window entries f16(code * f16(d))
+      const float dq = (float)(_Float16)d;
+      const uint2 w = uint2{pack_h2(qc[0] * dq, qc[1] * dq), pack_h2(qc[2] * dq, qc[3] * dq)};
+      if (si == 1) {
+        if (ok)
+          *reinterpret_cast<uint2 *>(reinterpret_cast<_Float16 *>(rp.win.k) +
+                                     ((size_t)kvh * rp.win.pad + rp.win.j0 + row) * hd + e) = w;
+      } else {
+        // back to one column per lane: column fcol + r16, tokens t0 .. t0+3
+        const uint2 wt = quad_t16(w.x, w.y, qj);
+        const int t0 = 16 * i + 4 * gg, cv = fcol + r16;
+        if (t0 >= a.m) continue;
+        _Float16 *vrow = reinterpret_cast<_Float16 *>(rp.win.vt) + (size_t)cv * rp.win.vst;
+        const int j = rp.win.j0 + t0;
+        if ((j & 3) == 0 && t0 + 3 < a.m) {
+          *reinterpret_cast<uint2 *>(vrow + window_vt_col(j)) = wt;  // 4 consecutive columns
+        } else {
+          const uint32_t ww[2] = {wt.x, wt.y};
+          for (int jj = 0; jj < 4 && t0 + jj < a.m; jj++)
+            reinterpret_cast<uint16_t *>(vrow)[window_vt_col(j + jj)] = (uint16_t)(ww[jj >> 1] >> (16 * (jj & 1)));
+        }
+      }
+    } else {
+      const int fcol = (NF == 1 ? 16 * u : UC * u + 16 * f);
+      if constexpr (EPI == EPI_F16 || EPI == EPI_F32) {
+        if (seg.bias) {
+          const float b = fcol + r16 < seg.n ? seg.bias[fcol + r16] : 0.0f;
+          v = float4{v.x + b, v.y + b, v.z + b, v.w + b};
+        }
+      }
+      const int col = fcol + cq4;
+      const bool in = row < a.m && col < seg.n;
+      if constexpr (EPI == EPI_F16) {
+        const uint2 w = quad_t16(pack_h2(v.x, v.y), pack_h2(v.z, v.w), qj);
+        if (in) {
           _Float16 *dst = reinterpret_cast<_Float16 *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col;
           if (((seg.ldo | seg.col0) & 3) == 0 && ((uintptr_t)seg.out & 7) == 0 && col + 4 <= seg.n) {
             *reinterpret_cast<uint2 *>(dst) = w;
@@ -303,146 +401,36 @@ __global__ __launch_bounds__(64 * max_waves(MT, NF)) void skinny_kernel(SkinnyAr
               reinterpret_cast<uint16_t *>(dst)[e] = (uint16_t)(ww[e >> 1] >> (16 * (e & 1)));
           }
         }
-      } else if constexpr (EPI == EPI_ROPE) {
-        // RoPE + Q8_0 K/V store: the values and rounding points of gemm_q4_0.hip's RoPE
-        // epilogue. Lanes 0-31 hold 32 columns of the first half of a head, lanes 32-63
-        // the columns head_dim/2 further: a Q8_0 block is half a wave, NeoX partners are
-        // lanes l and l ^ 32.
-        const GemmRope &rp = a.rope;
-        const int hd = rp.head_dim;
-        const bool neox = rp.mode != 0, rotate = si < 2;
-        const int fcol = rope_col(f);  // fragment's first column
-        const float b = seg.bias ? seg.bias[fcol + r16] : 0.0f;
-        const int col = fcol + cq4, e0 = col & (hd - 1);
-        float4 ca = ca0, cb = cb0;
-        if (rotate && (i0 > 0 || o != own0)) rope_cs(row, e0, ca, cb);
-        const uint2 xv = quad_t16(pack_h2(v.x + b, v.y + b), pack_h2(v.z + b, v.w + b), qj);
-        const half2v x01 = as_h2(xv.x), x23 = as_h2(xv.y);
-        const float x[4] = {(float)x01[0], (float)x01[1], (float)x23[0], (float)x23[1]};
-        float out[4] = {x[0], x[1], x[2], x[3]};
-        if (rotate && neox) {
-          const half2v p01 = as_h2((uint32_t)__shfl_xor((int)xv.x, 32, 64)), p23 = as_h2((uint32_t)__shfl_xor((int)xv.y, 32, 64));
-          const float p[4] = {(float)p01[0], (float)p01[1], (float)p23[0], (float)p23[1]};
-          const float cc[4] = {ca.x, ca.z, cb.x, cb.z}, ss[4] = {ca.y, ca.w, cb.y, cb.w};
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            out[j] = lane < 32 ? rot_sub(x[j], cc[j], p[j], ss[j]) : rot_add(p[j], ss[j], x[j], cc[j]);
-        } else if (rotate) {
-          const float cc[2] = {ca.x, ca.z}, ss[2] = {ca.y, ca.w};
-#pragma unroll
-          for (int j = 0; j < 4; j += 2) {
-            out[j] = rot_sub(x[j], cc[j / 2], x[j + 1], ss[j / 2]);
-            out[j + 1] = rot_add(x[j], ss[j / 2], x[j + 1], cc[j / 2]);
-          }
-        }
-        const bool ok = row < a.m;
-        if (si == 0) {
-          if (ok)
-            *reinterpret_cast<uint2 *>(reinterpret_cast<_Float16 *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col) =
-                uint2{pack_h2(out[0], out[1]), pack_h2(out[2], out[3])};
-          continue;
-        }
-        float amax = fmaxf(fmaxf(fabsf(out[0]), fabsf(out[1])), fmaxf(fabsf(out[2]), fabsf(out[3])));
-#pragma unroll
-        for (int sh = 4; sh <= 16; sh *= 2) amax = fmaxf(amax, __shfl_xor(amax, sh, 64));
-        const float d = amax / 127.0f;
-        const float id = d != 0.0f ? 1.0f / d : 0.0f;
-        float qc[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) qc[j] = fminf(fmaxf(roundf(out[j] * id), -128.0f), 127.0f);
-        const int kvh = head, e = e0;
-        if (ok) {
-          int slot_i = rp.slot0 + row;
-          if (slot_i >= rp.wrap) slot_i %= rp.wrap;
-          uint8_t *blk = (si == 1 ? rp.k_dst : rp.v_dst) + (size_t)slot_i * rp.row_bytes +
-                         (size_t)(kvh * (hd >> 5) + (e >> 5)) * 34;
-          if ((e & 31) == 0) *reinterpret_cast<_Float16 *>(blk) = (_Float16)d;
-          uint16_t *codes = reinterpret_cast<uint16_t *>(blk + 2 + (e & 31));  // 2-byte aligned
-#pragma unroll
-          for (int j = 0; j < 4; j += 2)
-            codes[j / 2] = (uint16_t)((uint8_t)(int8_t)(int)qc[j] | ((uint16_t)(uint8_t)(int8_t)(int)qc[j + 1] << 8));
-        }
-        if (!rp.win.k) continue;
-        // window entries f16(code * f16(d))
-        const float dq = (float)(_Float16)d;
-        const uint2 w = uint2{pack_h2(qc[0] * dq, qc[1] * dq), pack_h2(qc[2] * dq, qc[3] * dq)};
-        if (si == 1) {
-          if (ok)
-            *reinterpret_cast<uint2 *>(reinterpret_cast<_Float16 *>(rp.win.k) +
-                                       ((size_t)kvh * rp.win.pad + rp.win.j0 + row) * hd + e) = w;
-        } else {
-          // back to one column per lane: column fcol + r16, tokens t0 .. t0+3
-          const uint2 wt = quad_t16(w.x, w.y, qj);
-          const int t0 = 16 * i + 4 * gg, cv = fcol + r16;
-          if (t0 >= a.m) continue;
-          _Float16 *vrow = reinterpret_cast<_Float16 *>(rp.win.vt) + (size_t)cv * rp.win.vst;
-          const int j = rp.win.j0 + t0;
-          if ((j & 3) == 0 && t0 + 3 < a.m) {
-            *reinterpret_cast<uint2 *>(vrow + window_vt_col(j)) = wt;  // 4 consecutive columns
-          } else {
-            const uint32_t ww[2] = {wt.x, wt.y};
-            for (int jj = 0; jj < 4 && t0 + jj < a.m; jj++)
-              reinterpret_cast<uint16_t *>(vrow)[window_vt_col(j + jj)] = (uint16_t)(ww[jj >> 1] >> (16 * (jj & 1)));
-          }
-        }
       } else {
-        const int fcol = (NF == 1 ? 16 * u : UC * u + 16 * f);
-        if constexpr (EPI == EPI_F16 || EPI == EPI_F32) {
-          if (seg.bias) {
-            const float b = fcol + r16 < seg.n ? seg.bias[fcol + r16] : 0.0f;
-            v = float4{v.x + b, v.y + b, v.z + b, v.w + b};
+        if constexpr (EPI == EPI_RESID)  // x += f16(acc)
+          v = float4{(float)(_Float16)v.x, (float)(_Float16)v.y, (float)(_Float16)v.z, (float)(_Float16)v.w};
+        const float4 w = quad_t32(v.x, v.y, v.z, v.w, qj);
+        if (in) {
+          float *dst;
+          bool vec;
+          if constexpr (EPI == EPI_PART) {  // f32 partials, rows 4-column aligned (checked by the planner)
+            dst = a.part + ((size_t)ks * a.m + row) * a.ldp + colbase + col;
+            vec = col + 4 <= seg.n;
+          } else {
+            dst = reinterpret_cast<float *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col;
+            vec = ((seg.ldo | seg.col0) & 3) == 0 && ((uintptr_t)seg.out & 15) == 0 && col + 4 <= seg.n;
           }
-        }
-        const int col = fcol + cq4;
-        const bool in = row < a.m && col < seg.n;
-        if constexpr (EPI == EPI_F16) {
-          const uint2 w = quad_t16(pack_h2(v.x, v.y), pack_h2(v.z, v.w), qj);
-          if (in) {
-            _Float16 *dst = reinterpret_cast<_Float16 *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col;
-            if (((seg.ldo | seg.col0) & 3) == 0 && ((uintptr_t)seg.out & 7) == 0 && col + 4 <= seg.n) {
-              *reinterpret_cast<uint2 *>(dst) = w;
-            } else {
-              const uint32_t ww[2] = {w.x, w.y};
-              for (int e = 0; e < 4 && col + e < seg.n; e++)
-                reinterpret_cast<uint16_t *>(dst)[e] = (uint16_t)(ww[e >> 1] >> (16 * (e & 1)));
+          if (vec) {
+            float4 o4 = w;
+            if constexpr (EPI == EPI_RESID) {
+              const float4 old = *reinterpret_cast<const float4 *>(dst);
+              o4 = float4{old.x + w.x, old.y + w.y, old.z + w.z, old.w + w.w};
             }
-          }
-        } else {
-          if constexpr (EPI == EPI_RESID)  // x += f16(acc)
-            v = float4{(float)(_Float16)v.x, (float)(_Float16)v.y, (float)(_Float16)v.z, (float)(_Float16)v.w};
-          const float4 w = quad_t32(v.x, v.y, v.z, v.w, qj);
-          if (in) {
-            float *dst;
-            bool vec;
-            if constexpr (EPI == EPI_PART) {  // f32 partials, rows 4-column aligned (checked by the planner)
-              dst = a.part + ((size_t)ks * a.m + row) * a.ldp + colbase + col;
-              vec = col + 4 <= seg.n;
-            } else {
-              dst = reinterpret_cast<float *>(seg.out) + (size_t)row * seg.ldo + seg.col0 + col;
-              vec = ((seg.ldo | seg.col0) & 3) == 0 && ((uintptr_t)seg.out & 15) == 0 && col + 4 <= seg.n;
-            }
-            if (vec) {
-              float4 o4 = w;
-              if constexpr (EPI == EPI_RESID) {
-                const float4 old = *reinterpret_cast<const float4 *>(dst);
-                o4 = float4{old.x + w.x, old.y + w.y, old.z + w.z, old.w + w.w};
-              }
-              *reinterpret_cast<float4 *>(dst) = o4;
-            } else {
-              const float ww[4] = {w.x, w.y, w.z, w.w};
-              for (int e = 0; e < 4 && col + e < seg.n; e++) dst[e] = EPI == EPI_RESID ? dst[e] + ww[e] : ww[e];
-            }
+            *reinterpret_cast<float4 *>(dst) = o4;
+          } else {
+            const float ww[4] = {w.x, w.y, w.z, w.w};
+            for (int e = 0; e < 4 && col + e < seg.n; e++) dst[e] = EPI == EPI_RESID ? dst[e] + ww[e] : ww[e];
           }
         }
       }
     }
   }
 }
-
-struct SkinnyPlan {
-  int nf;      // weight fragments (16 rows) per wave
-  int splits;  // K splits across workgroups
-};
 
 int unit_cols_of(const GemmArgs &a, int nf) { return a.epi == EPI_SWIGLU ? 8 * nf : 16 * nf; }
 
@@ -456,7 +444,7 @@ int units_of(const GemmArgs &a, int nf) {
 int pairs_of(const GemmArgs &a) { return (a.k + kPairK - 1) / kPairK; }
 
 template <int MT, int NF, int EPI, bool SOA>
-int32_t launch_skinny_t(SkinnyArgs sa, int splits, hipStream_t s, LaunchStamp st) {
+int32_t launch_skinny_t(const SkinnyArgs &sa, int splits, hipStream_t s, LaunchStamp st) {
   // One step per wave where LDS holds the waves' X, the steps spread evenly over them
   // otherwise. Up to one workgroup per CU may take the CU's whole LDS. More workgroups
   // than CUs must run side by side (a second round costs the kernel's whole latency
@@ -464,13 +452,14 @@ int32_t launch_skinny_t(SkinnyArgs sa, int splits, hipStream_t s, LaunchStamp st
   // with six and 13.6 with twelve; 256 workgroups: 11.5 with twelve, 14.3 with four).
   const int slot = sa.xrows * kPairK * 2;
   const bool alone = sa.units * splits <= device_cu_count();
-  const size_t room = alone ? 156 << 10 : 76 << 10;
-  const int most = std::max(1, std::min({alone ? max_waves(MT, NF) : 4, (int)(room / slot)}));
+  constexpr int kRoomAlone = 156 << 10, kRoomShared = 76 << 10, kWavesShared = 4;
+  constexpr int kTiles = NF * MT * 1024;  // bytes of one wave's sums, which meet in LDS
+  static_assert(max_waves(MT, NF) * kTiles <= kRoomAlone && kWavesShared * kTiles <= kRoomShared, "the waves' sums fit");
+  const size_t room = alone ? kRoomAlone : kRoomShared;
+  const int most = std::max(1, std::min({alone ? max_waves(MT, NF) : kWavesShared, (int)(room / slot)}));
   const int iters = (sa.split_pairs + most - 1) / most;
   const int waves = (sa.split_pairs + iters - 1) / iters;
-  const size_t tile = (size_t)waves * NF * 1024;
-  sa.red_tiles = tile * MT <= room ? MT : 1;
-  const size_t lds = std::max((size_t)waves * slot, tile * sa.red_tiles);
+  const size_t lds = (size_t)waves * std::max(slot, kTiles);
   launch_stamped(skinny_kernel<MT, NF, EPI, SOA>, dim3((unsigned)sa.units, (unsigned)splits), dim3(64 * waves), lds, s,
                  st.start, st.stop, sa);
   const hipError_t e = hipGetLastError();
