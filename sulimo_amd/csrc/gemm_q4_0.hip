@@ -1578,12 +1578,12 @@ int32_t launch_gemm_q4_0(const GemmArgs &a, hipStream_t s, bool *norm_done, cons
       if (skinny) launch_stamped(k32, grid, block, 0, s, nullptr, st.stop, r);
       else launch_stamped(k16, grid, block, 0, s, nullptr, st.stop, r);
     };
-    switch (v4) {
+    switch (v4) {  // (skinny_splits: up to 4096 columns)
       case 1: norm(split_reduce_norm_kernel<1, false>, split_reduce_norm_kernel<1, true>); break;
       case 2: norm(split_reduce_norm_kernel<2, false>, split_reduce_norm_kernel<2, true>); break;
       case 3: norm(split_reduce_norm_kernel<3, false>, split_reduce_norm_kernel<3, true>); break;
       case 4: norm(split_reduce_norm_kernel<4, false>, split_reduce_norm_kernel<4, true>); break;
-      default: norm(split_reduce_norm_kernel<8, false>, split_reduce_norm_kernel<8, true>); break;
+      default: launch_stamped(split_reduce_norm_kernel<8, true>, grid, block, 0, s, nullptr, st.stop, r); break;
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "split_reduce_norm_kernel launch");

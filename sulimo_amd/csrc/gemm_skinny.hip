@@ -514,6 +514,9 @@ int skinny_splits(const GemmArgs &a, bool unbounded) {
   if (a.epi != EPI_RESID && a.epi != EPI_F16) return 1;
   for (int i = 0; i < a.nseg; i++)
     if (a.seg[i].n % 4 || a.seg[i].ldo % 4 || a.seg[i].col0 % 4) return 1;
+  // the reductions of f32 partials with the norm hold rows of up to 4096 columns (256 CUs
+  // leave no wider matrix a split)
+  if (a.epi == EPI_RESID && a.seg[0].n > 4096) return 1;
   const int pairs = pairs_of(a);
   int splits = std::min({kMaxSplits, device_cu_count() / std::max(1, units_of(a, 2)), (pairs + 2) / 3});
   if (splits < 2 || (a.epi == EPI_F16 && (a.m <= 16 || pairs < 32 || splits < 4))) return 1;

@@ -73,6 +73,7 @@ def run_mode(ctx, hm, toks, chunks, cap, unfused):
         c = hm.cfg
         snaps.append(dict(
             q=sb["q"].download(np.uint16, (m, c.q_dim)),
+            x=sb["x"].download(np.float16, (m, c.embd)),
             swiglu=sb["ffn_swiglu"].download(np.uint16, (m, c.ffn)),
             v=sb["v"].download(np.float16, (m, c.kv_dim)) if unfused else None,
             gate=sb["ffn_gate"].download(np.float16, (m, c.ffn)) if unfused else None,

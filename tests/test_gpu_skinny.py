@@ -74,6 +74,28 @@ def test_epilogues_bit_exact_vs_separate_kernels(ctx, cfg, chunks, cap):
         assert np.max(np.abs(f["logits"] - p["logits"])) <= 1e-3 * np.abs(p["logits"]).max()
 
 
+@pytest.mark.parametrize("D", [288, 1056, 2080, 3104])
+@pytest.mark.parametrize("n", [5, 33])
+def test_split_reduction_of_widths_not_256(ctx, D, n):
+    """Rows of 1 to 4 times 1024 columns, none a multiple of 256: the o and down projections
+    split k, and their reduction adds the f32 partials, updates the residual and norms the
+    row in a workgroup of its own. Against the separate kernels: the SwiGLU bytes (the FFN
+    norm of the o projection's rows), the final residual, the logits (the output norm)."""
+    cfg = S.ModelConfig(1, D, 1056, 8, 2, 64, 64, 512, 1e6, 1e-6, 1)
+    hm = exact_model(cfg, D + n)
+    toks = S.random_tokens(19, n, cfg.vocab)
+    print(f"split reduction: width {D}, {n} tokens", flush=True)
+    (f,), _ = run_mode(ctx, hm, toks, [n], 64, unfused=False)
+    (p,), _ = run_mode(ctx, hm, toks, [n], 64, unfused=True)
+    assert np.array_equal(f["swiglu"], p["swiglu"])
+    # the down projection's f16 value may round one step apart (it differs from x by the
+    # embedding, +-1), then x itself
+    x = np.abs(p["x"])
+    step = np.spacing(x + np.float16(1)).astype(np.float64) + np.spacing(x).astype(np.float64)
+    assert np.all(np.abs(f["x"].astype(np.float64) - p["x"].astype(np.float64)) <= step)
+    assert np.max(np.abs(f["logits"] - p["logits"])) <= 1e-3 * np.abs(p["logits"]).max()
+
+
 @pytest.mark.parametrize("M,k,m_out", [(5, 32, 8), (16, 1536, 1536), (24, 96, 40), (33, 2080, 264), (64, 416, 9000),
                                        (8, 4128, 72)])
 def test_no_alloc_reads_the_source_arrays(ctx, M, k, m_out):
