@@ -1,12 +1,13 @@
 """GPU: the allocation-free GEMM entry point (sulimo_hip_enqueue_gemm_q4_0_f16_noalloc)
 against the allocating one (sulimo_hip_enqueue_gemm_q4_0_f16) through the C ABI.
 
-Its scratch (the weights' GEMM layout and the K-split partial sums) is the library's
-static per-device array, which keeps the previous call's contents: two calls in a
-row, the second with smaller operands, and the first shape again after it, must each
-equal the allocating entry point's output bit for bit (same kernels, same plan), and
-stay within the oracle's error bound. A matrix too large for the array is refused on
-the host.
+Up to 4 tokens, and from some tens of tokens on, its scratch (the weights' GEMM layout and
+the K-split partial sums) is the library's static per-device array, which keeps the
+previous call's contents: calls in a row, the later ones with smaller operands, and the
+first shape again after them, must each equal the allocating entry point's output bit for
+bit (same kernels, same plan), and stay within the oracle's error bound. In between (5 to
+64 tokens of a matrix that is not too wide) the weights are read where they are and the
+array is left alone. A matrix too large for the array is refused on the host.
 """
 import ctypes
 
@@ -30,8 +31,9 @@ def _operands(ctx, seed, m_out, k, n_tok):
 
 
 def test_noalloc_gemm_matches_allocating_entry_point(ctx):
-    # (m_out, k, n_tok): the up-projection GEMM at 128 tokens, then a smaller one
-    shapes = [(8960, 1536, 128), (1536, 1536, 37), (8960, 1536, 128)]
+    # (m_out, k, n_tok): the up-projection GEMM at 128 tokens, one that leaves the array
+    # alone, smaller ones in the array (a tiled GEMM, a GEMV), the first again
+    shapes = [(8960, 1536, 128), (1536, 1536, 37), (1536, 1536, 300), (264, 416, 3), (8960, 1536, 128)]
     ops = {}
     for i, (m_out, k, n_tok) in enumerate(shapes):
         print(f"no-alloc GEMM call {i}: m_out {m_out} k {k} n_tok {n_tok}", flush=True)
@@ -63,21 +65,22 @@ def _free_device_bytes():
     return free.value
 
 
-def test_noalloc_gemm_allocates_nothing(ctx):
+@pytest.mark.parametrize("n_tok,n2", [(64, 37), (300, 257)], ids=["weights_in_place", "scratch"])
+def test_noalloc_gemm_allocates_nothing(ctx, n_tok, n2):
     """The device's free memory is unchanged by two no-alloc calls on freshly uploaded
     weights (24.8 MB in the GEMM layout, which the allocating entry point would build
     and cache), and the allocating call that follows does lower it: the probe sees an
     allocation of that size. Two contexts, each on its own stream, then call the entry
-    point back to back: the library orders them, and both outputs equal the allocating
-    entry point's."""
-    m_out, k, n_tok = 28672, 1536, 64
+    point back to back, a large matrix and then a small one: where they share the scratch
+    array the library orders them, and both outputs equal the allocating entry point's."""
+    m_out, k = 28672, 1536
     t, x, (sb, qb, xb) = _operands(ctx, 300, m_out, k, n_tok)
     outs = [hip.HipBuffer.device_only(ctx, n_tok * m_out * 2) for _ in range(3)]
-    t2, x2, (sb2, qb2, xb2) = _operands(ctx, 310, 1536, 1536, 37)
-    o2 = hip.HipBuffer.device_only(ctx, 37 * 1536 * 2)
-    o2_ref = hip.HipBuffer.device_only(ctx, 37 * 1536 * 2)
-    # a first call loads the kernels' code objects (run alone, this test is their first user)
-    hip.enqueue_gemm_q4_0_f16_noalloc(ctx, sb2, qb2, xb2, o2, 1536, 1536, 37)
+    t2, x2, (sb2, qb2, xb2) = _operands(ctx, 310, 1536, 1536, n2)
+    o2 = hip.HipBuffer.device_only(ctx, n2 * 1536 * 2)
+    o2_ref = hip.HipBuffer.device_only(ctx, n2 * 1536 * 2)
+    # first calls load the kernels' code objects (run alone, this test is their first user)
+    hip.enqueue_gemm_q4_0_f16_noalloc(ctx, sb2, qb2, xb2, o2, 1536, 1536, n2)
     ctx.wait()
     before = _free_device_bytes()
     hip.enqueue_gemm_q4_0_f16_noalloc(ctx, sb, qb, xb, outs[0], m_out, k, n_tok)
@@ -96,15 +99,15 @@ def test_noalloc_gemm_allocates_nothing(ctx):
     other = hip.HipContext.new(0)
     try:
         hip.enqueue_gemm_q4_0_f16_noalloc(ctx, sb, qb, xb, outs[0], m_out, k, n_tok)
-        hip.enqueue_gemm_q4_0_f16_noalloc(other, sb2, qb2, xb2, o2, 1536, 1536, 37)
+        hip.enqueue_gemm_q4_0_f16_noalloc(other, sb2, qb2, xb2, o2, 1536, 1536, n2)
         other.wait()
         ctx.wait()
     finally:
         other.release()
-    hip.enqueue_gemm_q4_0_f16(ctx, sb2, qb2, xb2, o2_ref, 1536, 1536, 37)
+    hip.enqueue_gemm_q4_0_f16(ctx, sb2, qb2, xb2, o2_ref, 1536, 1536, n2)
     ctx.wait()
     assert np.array_equal(outs[0].download(np.uint16, (n_tok, m_out)), want)
-    assert np.array_equal(o2.download(np.uint16, (37, 1536)), o2_ref.download(np.uint16, (37, 1536)))
+    assert np.array_equal(o2.download(np.uint16, (n2, 1536)), o2_ref.download(np.uint16, (n2, 1536)))
     for b in (sb, qb, xb, sb2, qb2, xb2, o2, o2_ref, *outs):
         b.release()
 
