@@ -144,10 +144,10 @@ int32_t sulimo_hip_enqueue_gemm_q4_0_f16(sulimo_hip_ctx *ctx, const sulimo_hip_b
  * in a static device array of 64 MiB that every GPU the library runs on holds until
  * the process ends. Matrices whose layout exceeds it (m * k * 18/32 bytes, rounded up
  * to 32 rows and 64 columns) are rejected with SULIMO_HIP_ERR_INVALID_ARGUMENT. All
- * calls on one GPU share that array, so the library orders them: each call's stream
- * first waits for an event the previous no-alloc call on that GPU recorded, from
- * whichever context or thread it came. Calls from two streams therefore run one after
- * the other, never at once. */
+ * calls on one GPU share that array (calls of 5 to 64 tokens of a matrix that is not too
+ * wide read the weights where they are instead), so the library orders them: a call first
+ * waits for the previous no-alloc call on that GPU, from whichever context or thread it
+ * came. Calls from two streams therefore run one after the other, never at once. */
 int32_t sulimo_hip_enqueue_gemm_q4_0_f16_noalloc(sulimo_hip_ctx *ctx, const sulimo_hip_buffer *scales,
                                                  const sulimo_hip_buffer *quants,
                                                  const sulimo_hip_buffer *x, sulimo_hip_buffer *out,

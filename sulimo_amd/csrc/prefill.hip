@@ -177,19 +177,19 @@ int32_t sulimo_hip_enqueue_gemm_q4_0_f16_noalloc(sulimo_hip_ctx *ctx, const suli
   a.epi = EPI_F16;
   a.seg[0] = GemmSegment{nullptr, out->dev, (int)m, (int)m, 0};
   a.nseg = 1;
-  // A handful of tokens (more than the GEMV's 4): the skinny kernel reads the weights where
-  // they are, in one launch, and leaves the scratch array alone (1536 x 1536 at 16 tokens:
-  // 15.5 us with the pack, the event and the tiled kernel, 4.6 so).
-  if (n > 4 && skinny_fits(a)) {
-    wrote(out);
-    return launch_skinny_soa(a, dp<const uint16_t>(scales), dp<const uint8_t>(quants), ctx->stream);
-  }
   NoAllocOrder *order = noalloc_order(ctx->device);
   if (!order) return fail(SULIMO_HIP_ERR_DRIVER, "the no-alloc ordering event was not created");
   // After the previous no-alloc call on this device, from whatever stream it came.
   std::lock_guard<std::mutex> serial(order->m);
-  SULIMO_HIP_TRY(hipStreamWaitEvent(ctx->stream, order->ev, 0));
+  if ((rc = order->begin(ctx->stream))) return rc;
   wrote(out);
+  // A handful of tokens (more than the GEMV's 4): the skinny kernel reads the weights where
+  // they are, in one launch, and leaves the scratch array alone (1536 x 1536 at 16 tokens:
+  // 15.5 us with the pack, the event and the tiled kernel, 4.6 so).
+  if (n > 4 && skinny_fits(a)) {
+    if ((rc = launch_skinny_soa(a, dp<const uint16_t>(scales), dp<const uint8_t>(quants), ctx->stream))) return rc;
+    return order->end(ctx->stream);
+  }
   uint8_t *scr = reinterpret_cast<uint8_t *>(ctx->scratch);
   if ((rc = launch_pack_q4_panels(dp<const uint16_t>(scales), dp<const uint8_t>(quants), nullptr, nullptr, (int)m,
                                   (int)k, scr, ctx->stream)))
@@ -198,8 +198,7 @@ int32_t sulimo_hip_enqueue_gemm_q4_0_f16_noalloc(sulimo_hip_ctx *ctx, const suli
   a.part = reinterpret_cast<float *>(scr + pan_al);
   a.part_bytes = kNoAllocScratchBytes - pan_al;
   if ((rc = launch_gemm_q4_0(a, ctx->stream))) return rc;
-  SULIMO_HIP_TRY(hipEventRecord(order->ev, ctx->stream));
-  return SULIMO_HIP_OK;
+  return order->end(ctx->stream);
 }
 
 int32_t sulimo_hip_gemm_q4_0_f16(sulimo_hip_ctx *ctx, const sulimo_hip_buffer *scales,
@@ -939,6 +938,9 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
       if (g.key == key) hit = &g;
     if (!hit) {
       hipGraph_t g1 = nullptr, g2 = nullptr;
+      // (no other context's no-alloc call may record its event on a stream under capture)
+      std::unique_lock<std::mutex> no_record;
+      if (NoAllocOrder *order = noalloc_order(ctx->device)) no_record = std::unique_lock<std::mutex>(order->m);
       SULIMO_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       bool split = false;
       int32_t brc = body([&]() -> int32_t {
@@ -952,6 +954,7 @@ int32_t sulimo_hip_execute_prefill_ubatch_ex(
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       hipError_t ce = hipStreamIsCapturing(s, &cs);
       if (ce == hipSuccess && cs != hipStreamCaptureStatusNone) ce = hipStreamEndCapture(s, &g2);
+      if (no_record) no_record.unlock();
       PrefillGraph pg;
       pg.key = std::move(key);
       if (brc == SULIMO_HIP_OK && ce == hipSuccess && split && g1 && g2) {

@@ -160,6 +160,25 @@ NoAllocOrder *noalloc_order(int device) {
   return device >= 0 && device < 64 && g_noalloc_order[device].ev ? &g_noalloc_order[device] : nullptr;
 }
 
+int32_t NoAllocOrder::begin(hipStream_t s) {
+  if (last && last != s) {
+    if (!recorded) SULIMO_HIP_TRY(hipEventRecord(ev, last));
+    recorded = true;
+    SULIMO_HIP_TRY(hipStreamWaitEvent(s, ev, 0));
+  }
+  last = s;
+  recorded = false;
+  return SULIMO_HIP_OK;
+}
+
+int32_t NoAllocOrder::end(hipStream_t s) {
+  if (contexts > 1) {
+    SULIMO_HIP_TRY(hipEventRecord(ev, s));
+    recorded = true;
+  }
+  return SULIMO_HIP_OK;
+}
+
 // Per-device address of `scratch`, resolved once per device with that device current,
 // and the event that orders the no-alloc calls on it.
 static int32_t resolve_scratch(int device, void **out) {
@@ -218,6 +237,10 @@ static int32_t create_ctx(int device, bool shared, sulimo_hip_ctx **out) {
     hipStreamDestroy(c->side);
     delete c;
     return rc;
+  }
+  if (NoAllocOrder *order = noalloc_order(device)) {
+    std::lock_guard<std::mutex> g(order->m);
+    order->contexts++;
   }
   *out = c;
   return SULIMO_HIP_OK;
@@ -314,6 +337,11 @@ int32_t sulimo_hip_context_release(sulimo_hip_ctx *ctx) {
   if (!ctx || ctx->shared) return SULIMO_HIP_OK;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->stream);
+  if (NoAllocOrder *order = noalloc_order(ctx->device)) {  // (its calls have ended)
+    std::lock_guard<std::mutex> g(order->m);
+    if (order->last == ctx->stream) order->last = nullptr;
+    order->contexts--;
+  }
   if (ctx->ws) hipFree(ctx->ws);
   if (ctx->tok) hipFree(ctx->tok);
   if (ctx->attn_ctr) hipFree(ctx->attn_ctr);

@@ -112,6 +112,48 @@ def test_noalloc_gemm_allocates_nothing(ctx, n_tok, n2):
         b.release()
 
 
+def test_noalloc_calls_of_two_contexts_run_in_order(ctx):
+    """A call reads what another context's no-alloc call writes, with no wait in between:
+    behind some milliseconds of calls on the first context's stream, from a second context
+    that is made after them, and from one that is there already; where the weights are read
+    in place (16 tokens), in the scratch array (130) and from the one to the other."""
+    big, d, pairs = (28672, 1536, 64), 1536, [(16, 16), (130, 130), (16, 130), (130, 16)]
+    _, _, fill = _operands(ctx, 400, *big)
+    fill_out = hip.HipBuffer.device_only(ctx, big[2] * big[0] * 2)
+    w1, w2 = (S.random_q4(np.random.default_rng(410 + i), d, d) for i in range(2))
+    (s1, q1), (s2, q2) = ([hip.HipBuffer.from_host(ctx, a, True) for a in (w.scales, w.quants)] for w in (w1, w2))
+    other = None
+    try:
+        for na, nb in pairs:
+            n = max(na, nb)
+            xb = hip.HipBuffer.from_host(ctx, S.random_activations(420, (n, d)), True)
+            mid, ref, want, got = (hip.HipBuffer.from_host(ctx, np.zeros((n, d), np.float16)) for _ in range(4))
+            hip.enqueue_gemm_q4_0_f16(ctx, s1, q1, xb, ref, d, d, na)
+            hip.enqueue_gemm_q4_0_f16(ctx, s2, q2, ref, want, d, d, nb)
+            ctx.wait()
+            print(f"no-alloc order: {na} then {nb} tokens", flush=True)
+            for _ in range(300):
+                hip.enqueue_gemm_q4_0_f16_noalloc(ctx, *fill, fill_out, *big)
+            hip.enqueue_gemm_q4_0_f16_noalloc(ctx, s1, q1, xb, mid, d, d, na)
+            other = other or hip.HipContext.new(0)
+            hip.enqueue_gemm_q4_0_f16_noalloc(other, s2, q2, mid, got, d, d, nb)
+            other.wait()
+            ctx.wait()
+            assert np.array_equal(got.download(np.uint16, (n, d)), want.download(np.uint16, (n, d))), (na, nb)
+            for b in (xb, mid, ref, want, got):
+                b.release()
+    finally:
+        if other:
+            other.release()
+    # calls go on after the other context is gone
+    o = hip.HipBuffer.device_only(ctx, big[2] * big[0] * 2)
+    hip.enqueue_gemm_q4_0_f16_noalloc(ctx, *fill, o, *big)
+    ctx.wait()
+    assert np.array_equal(o.download(np.uint16, (big[2], big[0])), fill_out.download(np.uint16, (big[2], big[0])))
+    for b in (*fill, fill_out, o, s1, q1, s2, q2):
+        b.release()
+
+
 def test_noalloc_gemm_rejects_matrices_beyond_the_scratch(ctx):
     """The LM head (151936 x 1536: 131 MB in the GEMM layout) exceeds the 64 MiB array:
     refused before anything is launched."""
