@@ -1198,8 +1198,9 @@ int32_t launch_gemv_mt(const GemmArgs &args, hipStream_t s, LaunchStamp st) {
   GemmArgs a = args;
   int panels = 0;
   for (int i = 0; i < a.nseg; i++) panels += (a.seg[i].n + 31) / 32;
-  // waves per panel: enough for eight waves per CU, at least two stages each (1536 x 8960
-  // at one token 37.6 -> 8.7 us, 8960 x 1536 8.7 -> 5.6); a wide matrix fills the CUs as it is
+  // waves per panel: a power of two, enough for eight waves per CU, two stages each or more
+  // on average (runs are rounded up, so the last waves of a panel may hold none); 1536 x 8960
+  // at one token 37.6 -> 8.7 us, 8960 x 1536 8.7 -> 5.6; a wide matrix fills the CUs as it is
   const int nst = (a.k / 32 + 1) / 2;
   a.splits = 1;
   while (a.splits < kGemvMaxSplits && panels * a.splits < 8 * device_cu_count() && nst >= 4 * a.splits) a.splits *= 2;

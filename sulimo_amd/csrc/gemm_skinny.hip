@@ -448,8 +448,9 @@ int32_t launch_skinny_t(const SkinnyArgs &sa, int splits, hipStream_t s, LaunchS
   // One step per wave where LDS holds the waves' X, the steps spread evenly over them
   // otherwise. Up to one workgroup per CU may take the CU's whole LDS. More workgroups
   // than CUs must run side by side (a second round costs the kernel's whole latency
-  // again): four waves each (gate/up of 280 workgroups at m = 23: 10.9 us against 12.7
-  // with six and 13.6 with twelve; 256 workgroups: 11.5 with twelve, 14.3 with four).
+  // again): four waves each (gate/up of 280 workgroups: at 23 tokens 9.6 us against 11.2
+  // with six and 12.7 with twelve, at 40 tokens 11.4 against 14.7; of 256 workgroups: at 23
+  // tokens 10.2 with twelve and 12.2 with four, at 40 12.4 and 14.7).
   const int slot = sa.xrows * kPairK * 2;
   const bool alone = sa.units * splits <= device_cu_count();
   constexpr int kRoomAlone = 156 << 10, kRoomShared = 76 << 10, kWavesShared = 4;
@@ -491,9 +492,12 @@ SkinnyArgs skinny_args(const GemmArgs &a, int nf, int *splits) {
 
 // Token counts and widths the skinny kernel takes from the tiled one: up to 64 tokens (48
 // with the RoPE epilogue, whose units of 64 columns leave few workgroups: 12.7 us against
-// 11.4 tiled at 64, 11.0 against 11.5 at 48), and few enough columns that a unit of 64
-// leaves at most two workgroups per CU (beyond that each CU would read X again and again,
-// and the tiles of the other kernel fill the chip).
+// 11.4 tiled at 64, 11.0 against 11.5 at 48; at 64 tokens the others still gain, the two
+// models' shapes: gate/up 13.9 and 14.8 us against 17.3 and 27.0 tiled, o and down with
+// their norm 10.2 to 18.5 against 10.8 to 21.9, single f16 projections 6.0 to 14.9 against
+// 9.0 to 15.1; more tokens than four tiles of 16 rows are not built), and few enough
+// columns that a unit of 64 leaves at most two workgroups per CU (beyond that each CU would
+// read X again and again, and the tiles of the other kernel fill the chip).
 bool skinny_fits(const GemmArgs &a) {
   if (a.m < 1 || a.m > kSkinnyMaxTokens || a.ldx % 8) return false;
   if (a.epi == EPI_ROPE) {

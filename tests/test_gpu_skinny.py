@@ -31,6 +31,18 @@ def test_ragged(ctx, M, k, m_out):
     assert np.all(np.abs(y.astype(np.float64) - ref) <= f16_weight_bound(x, w.scales, w.quants, ref))
 
 
+@pytest.mark.parametrize("M,k", [(1, 33024), (2, 16480), (3, 8960), (4, 8224)])
+def test_gemv_tokens_beyond_its_lds(ctx, M, k):
+    """Up to 4 tokens of a k whose activations exceed the GEMV's 64 KB of LDS come here too."""
+    rng = np.random.default_rng(M)
+    w = S.random_q4(rng, 72, k)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    print(f"skinny GEMM m={M} k={k} n=72", flush=True)
+    y = run_gemm(ctx, w.scales, w.quants, x, 72, k, M)
+    ref = oracle.gemm_q4_0_f16_scalar_reference(w.scales, w.quants, x, 72, k, M)
+    assert np.all(np.abs(y.astype(np.float64) - ref) <= f16_weight_bound(x, w.scales, w.quants, ref))
+
+
 @pytest.mark.parametrize("M", [7, 23, 32])
 @pytest.mark.parametrize("k,m_out", [(1536, 1536), (1536, 8960), (8960, 1536), (3072, 8192), (8192, 3072)])
 def test_layer_shapes(ctx, M, k, m_out):
