@@ -8,6 +8,10 @@ argmax) with the tighter bounds of this build: logits max rel err <= 1e-2 of the
 logit scale, top-1 agreement >= 99.5 % over all positions.
 """
 import dataclasses
+import os
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -250,6 +254,72 @@ def test_graph_replay_bit_identical(layers, calls, cap):
         assert np.array_equal(lg.view(np.uint32), le.view(np.uint32)), f"logits of call {i}"
         for l in range(cfg.n_layers):
             assert np.array_equal(k[l], ke[l]) and np.array_equal(v[l], ve[l]), f"K/V of call {i}, layer {l}"
+
+
+# hipGraphInstantiate in front of the runtime's, found first because it is loaded first:
+# reports out of memory while `fail` is set.
+_INSTANTIATE_SHIM = """
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+int fail = 1, calls = 0;
+int hipGraphInstantiate(void **exec, void *graph, void **node, char *log, size_t size) {
+  calls++;
+  if (fail) return 2;
+  void *rt = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+  if (!rt) rt = dlopen("libamdhip64.so", RTLD_LAZY);
+  int (*real)(void **, void *, void **, char *, size_t) = rt ? dlsym(rt, "hipGraphInstantiate") : NULL;
+  return real ? real(exec, graph, node, log, size) : 1;
+}
+"""
+_FAILED_CAPTURE = """
+import ctypes, sys
+import numpy as np
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+from sulimo_amd import hip
+from sulimo_amd import synthetic as S
+fail, calls = (ctypes.c_int.in_dll(shim, n) for n in ("fail", "calls"))
+cfg = S.ModelConfig(5, 256, 512, 4, 2, 64, 64, 512, 1e6, 1e-6, 1)
+toks = S.random_tokens(5, 40, cfg.vocab)
+ctx = hip.HipContext.get_or_init(0)
+dm = hip.DeviceModel(ctx, S.make_model(cfg, 4), 64, 40)
+dm.embed(toks)
+x = dm.scratch_bufs["x"].download(np.uint16, (40, cfg.embd))
+try:
+    dm.execute_prefill_ubatch(0, 40)
+    raise SystemExit("the call did not report the failed capture")
+except hip.HipError as e:
+    print("refused:", e, flush=True)
+assert calls.value > 0
+ctx.wait()
+dm.kv_sync_to_host(0, 64)
+assert not any(a.any() for ring in dm.kv_host() for a in ring), "K/V written by a call that failed"
+assert np.array_equal(dm.scratch_bufs["x"].download(np.uint16, (40, cfg.embd)), x)
+fail.value = 0
+dm.execute_prefill_ubatch(0, 40)
+got = dm.logits()
+ctx.set_graph_replay(False)
+dm.embed(toks)
+dm.execute_prefill_ubatch(0, 40)
+assert np.array_equal(got, dm.logits())
+print("capture ok", flush=True)
+"""
+
+
+def test_failed_capture_launches_nothing(tmp_path):
+    """A call whose graphs cannot be instantiated returns the error with nothing of the
+    ubatch launched: the rings and the embeddings are what they were, and the next call,
+    whose capture works, gives the eager result."""
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc is not installed")
+    (tmp_path / "shim.c").write_text(_INSTANTIATE_SHIM)
+    (tmp_path / "run.py").write_text(_FAILED_CAPTURE)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "shim.c"), "-o", str(tmp_path / "shim.so"), "-ldl"], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(hip.__file__)))
+    path = os.pathsep.join([root] + [p for p in [os.environ.get("PYTHONPATH")] if p])
+    r = subprocess.run([sys.executable, str(tmp_path / "run.py"), str(tmp_path / "shim.so")], capture_output=True, text=True,
+                       timeout=100, cwd=root, env=dict(os.environ, PYTHONPATH=path))
+    assert r.returncode == 0 and "capture ok" in r.stdout, r.stdout + r.stderr
 
 
 def test_profiled_prefill_is_unchanged_and_counts_launches():
